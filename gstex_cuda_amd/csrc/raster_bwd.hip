@@ -9,6 +9,8 @@
 // values of the chart's route.  Using delta = l1*ax1 + l2*ax2 (the ray hits
 // the splat plane), each outer product sum_pixels v * delta becomes
 // ax1 * sum(v*l1) + ax2 * sum(v*l2).
+#include <type_traits>
+
 #include "raster_common.hpp"
 #include "sh_basis.hpp"
 
@@ -18,38 +20,39 @@ namespace gstex {
 // MODE 0 compiles out the blur (settings bit 9), NDC distortion (bit 10)
 // and float64 edge-on code for the common settings; MODE 1 keeps all of it;
 // MODE 2 is MODE 0 plus the float64 edge-on solve.  TB selects bfloat16
-// texels.  CM <= 4 is the exact channel count; above 4, CM bounds a runtime
-// count.  The plain kernels for CM <= 4 are held to 96 VGPRs (5 waves per
-// SIMD), which they need at most one register more than.
+// texels.  CM <= 4 is the exact channel count; above 4 it is a runtime count.
+// The plain kernels for CM <= 4 are held to 96 VGPRs (5 waves per SIMD), which
+// they need at most one register more than, those for a runtime count to 128.
 //
 // Texel gradients of the window route over the R x Q texels from chart row
 // ou, column ov (R, Q <= 3): window tap (row r, column q) has weight
 // A[r] * B[q], and rows and columns from R, Q on carry zero weight on every
-// valid lane.  One reduction of the R * Q * CM values; the lane holding a
+// valid lane.  One reduction of the R * Q * CV values of CV channels (rows of
+// `stride` channels, the first `limit` of the CV exist); the lane holding a
 // wave total adds it to its texel.
-template <int R, int Q, int CM>
+template <int R, int Q, int CV>
 __device__ __forceinline__ void window_texel_add(const float (&A)[3], const float (&B)[3],
-                                                 const float (&vval)[CM], int lane,
+                                                 const float (&vval)[CV], int lane,
                                                  float* vtex_chart, int ou, int ov, int h,
-                                                 int w) {
-    float vals[R * Q * CM];
+                                                 int w, int stride, int limit) {
+    float vals[R * Q * CV];
 #pragma unroll
     for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
             const float ab = A[r] * B[q];
 #pragma unroll
-            for (int c = 0; c < CM; ++c) vals[(Q * r + q) * CM + c] = ab * vval[c];
+            for (int c = 0; c < CV; ++c) vals[(Q * r + q) * CV + c] = ab * vval[c];
         }
     const float tot = wave_reduce_scatter(vals, lane);
-    const int code = rs_slot<R * Q * CM>(lane);
+    const int code = rs_slot<R * Q * CV>(lane);
     if (code < 64 && tot != 0.f) {
-        const int rq = code / CM, c = code - CM * rq;
+        const int rq = code / CV, c = code - CV * rq;
         const int r = rq / Q, q = rq - Q * r;
         // a window row or column past the chart edge carries no weight
         // (taps clamp inside the chart)
-        if (ou + r < h && ov + q < w)
-            unsafeAtomicAdd(vtex_chart + ((ou + r) * w + (ov + q)) * CM + c, tot);
+        if (ou + r < h && ov + q < w && (limit >= CV || c < limit))
+            unsafeAtomicAdd(vtex_chart + ((ou + r) * w + (ov + q)) * stride + c, tot);
     }
 }
 
@@ -66,6 +69,150 @@ __device__ __forceinline__ void window_weights(float w0, float w1, int i, int j,
     W[0] = at0 ? first : 0.f;
     W[1] = at0 ? second : first;
     W[2] = at0 ? 0.f : second;
+}
+
+// CM of the kernels for more than four channels: the count is a runtime value.
+constexpr int kRuntimeCM = 8;
+
+// Channels cb .. cb + 3 of a pixel's texture cotangent (its row `src` of C
+// values), zero past C.  The kernels for a runtime count read them again for
+// every entry: the reads of a wave hit L1, and a register per channel would
+// cost the waves in flight.
+__device__ __forceinline__ void cotangents4(const float* src, int C, int cb, float (&v)[4]) {
+    if (cb + 4 <= C) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v[c] = src[cb + c];
+    } else {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v[c] = cb + c < C ? src[cb + c] : 0.f;
+    }
+}
+
+// Texel gradients of a chart with a runtime count C of more than four
+// channels; cot is this pixel's row of texture cotangents.  The routes are those of the exact channel counts, over
+// groups of four channels: a group's reduction sums its values over the wave,
+// so a texel takes one atomic per channel however many lanes sample it.
+//   single  1x1 chart
+//   quad    every valid lane samples one texel quad: 4 taps x 4 channels
+//   window  every valid lane's taps inside one 3x3 window (2x3, 3x2 where
+//           its last row or column is out of reach)
+//   lds     charts of up to kTexAccFloats values: lanes on one quad merged,
+//           then LDS adds and a flush
+//   direct  one atomic per tap and channel of the merged lanes
+// Bound by instruction issue, like the exact counts.  Before, every such chart
+// took per-lane LDS or global atomics, which serialise where the lanes of a
+// wave meet on one texel: a pass over 50k Gaussians at 800 x 600 with 8
+// channels took 4.9 ms, and 1.46 ms with these routes.
+__device__ __forceinline__ void texel_gradients_wide(
+    const float* cot, int C, float vis, const float (&wt)[4], const int (&lofs)[4], float fu,
+    float fv, int iu, int iv, int ju, int jv, bool bilinear, bool valid, uint64_t vmask, int hw,
+    int h, int w, int lane, float* acc, float* vtex_chart) {
+    const int first = __ffsll((unsigned long long)vmask) - 1;
+    if (hw == 1) {
+        const float ws = vis * ((wt[0] + wt[1]) + (wt[2] + wt[3]));
+        const int code = rs_slot<4>(lane);
+        for (int cb = 0; cb < C; cb += 4) {
+            float v[4];
+            cotangents4(cot, C, cb, v);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[c] *= ws;
+            const float tot = wave_reduce_scatter(v, lane);
+            if (code < 64 && cb + code < C && tot != 0.f)
+                unsafeAtomicAdd(vtex_chart + cb + code, tot);
+        }
+        return;
+    }
+    const int l0 = __builtin_amdgcn_readlane(lofs[0], first);
+    if (!(lanes_where(lofs[0] != l0) & vmask)) {
+        const int l1 = __builtin_amdgcn_readlane(lofs[1], first);
+        const int l2 = __builtin_amdgcn_readlane(lofs[2], first);
+        const int l3 = __builtin_amdgcn_readlane(lofs[3], first);
+        float wv[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) wv[k] = wt[k] * vis;
+        const int code = rs_slot<16>(lane);
+        const int k = code >> 2, cc = code & 3;
+        const int at = k == 0 ? l0 : k == 1 ? l1 : k == 2 ? l2 : l3;
+        for (int cb = 0; cb < C; cb += 4) {
+            float v[4], vals[16];
+            cotangents4(cot, C, cb, v);
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) vals[4 * t + c] = wv[t] * v[c];
+            const float tot = wave_reduce_scatter(vals, lane);
+            if (code < 64 && cb + cc < C && tot != 0.f)
+                unsafeAtomicAdd(vtex_chart + at + cb + cc, tot);
+        }
+        return;
+    }
+    if (bilinear) {
+        // window origin: the anchor lane's tap row / column, one lower when
+        // some valid lane lies below it
+        const int au = __builtin_amdgcn_readlane(iu, first);
+        const int av = __builtin_amdgcn_readlane(iv, first);
+        const int ou = au - ((lanes_where(iu < au) & vmask) ? 1 : 0);
+        const int ov = av - ((lanes_where(iv < av) & vmask) ? 1 : 0);
+        const int ri = iu - ou, rj = ju - ou, ci = iv - ov, cj = jv - ov;
+        if (!(lanes_where(((uint32_t)ri | (uint32_t)ci) > 1u) & vmask)) {
+            float A[3], B[3];
+            window_weights(1.f - fu, fu, ri, rj, A);
+            window_weights(1.f - fv, fv, ci, cj, B);
+#pragma unroll
+            for (int r = 0; r < 3; ++r) A[r] *= vis;
+            auto window = [&](auto R, auto Q) {
+                for (int cb = 0; cb < C; cb += 4) {
+                    float v[4];
+                    cotangents4(cot, C, cb, v);
+                    window_texel_add<R.value, Q.value, 4>(A, B, v, lane, vtex_chart + cb, ou, ov,
+                                                          h, w, C, C - cb);
+                }
+            };
+            using two = std::integral_constant<int, 2>;
+            using three = std::integral_constant<int, 3>;
+            if (!(lanes_where(rj == 2) & vmask)) window(two{}, three{});
+            else if (!(lanes_where(cj == 2) & vmask)) window(three{}, two{});
+            else window(three{}, three{});
+            return;
+        }
+    }
+    const QuadMerge qm = quad_merge_setup(valid ? lofs[0] : -1, lane);
+    const bool lds = hw * C <= kTexAccFloats;
+    for (int cb = 0; cb < C; cb += 4) {
+        float v[4];
+        cotangents4(cot, C, cb, v);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            float q[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) q[k] = quad_merge(wt[k] * (vis * v[c]), qm);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (q[k] == 0.f || cb + c >= C) continue;
+                if (lds) atomicAdd(acc + lofs[k] + cb + c, q[k]);
+                else unsafeAtomicAdd(vtex_chart + lofs[k] + cb + c, q[k]);
+            }
+        }
+    }
+    if (!lds) return;
+    // flush only the texels some valid lane touched
+    int lo = 0x7fffffff, hi = -1;
+    if (valid) {
+        lo = min(min(lofs[0], lofs[1]), min(lofs[2], lofs[3]));
+        hi = max(max(lofs[0], lofs[1]), max(lofs[2], lofs[3]));
+    }
+    lo = wave_min(lo);
+    hi = wave_max(hi);
+    // every lane's LDS adds precede these reads in the wave's LDS queue
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (int k = lo + lane; k < hi + C; k += kWave) {
+        const float v = acc[k];
+        if (v != 0.f) {
+            unsafeAtomicAdd(vtex_chart + k, v);
+            acc[k] = 0.f;
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
 }
 
 // raster_backward_wave runs one wave's share of a tile (wave `wave` of the
@@ -95,9 +242,10 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
     float T = 1.f, S0 = 0.f, S1 = 0.f, S2 = 0.f, vdep = 0.f, vreg = 0.f, vT = 0.f;
     V3 vo = v3(0.f, 0.f, 0.f), vn = v3(0.f, 0.f, 0.f);
     int dfin = -1, bfin = -1;
-    float vtex[CM];
+    const float* const cot = b.v_texture_out + (size_t)pid * C;
+    float vtex[CM <= 4 ? CM : 1];  // more than four stay in memory (cotangents4)
 #pragma unroll
-    for (int c = 0; c < CM; ++c) vtex[c] = 0.f;
+    for (int c = 0; c < (CM <= 4 ? CM : 1); ++c) vtex[c] = 0.f;
     if (inside) {
         T = b.final_Ts[pid];
         S0 = b.final_s[3 * pid];
@@ -109,9 +257,10 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
         vn = v3(b.v_normal[3 * pid], b.v_normal[3 * pid + 1], b.v_normal[3 * pid + 2]);
         vdep = b.v_depth[pid];
         vreg = b.v_reg[pid];
+        if constexpr (CM <= 4) {
 #pragma unroll
-        for (int c = 0; c < CM; ++c)
-            if (c < C) vtex[c] = b.v_texture_out[(size_t)pid * C + c];
+            for (int c = 0; c < CM; ++c) vtex[c] = cot[c];
+        }
         if constexpr (CM == 3) {
             if (b.loss_target) {  // vo, vtex hold out_img, out_texture
                 const float* tg = b.loss_target + 3 * pid;
@@ -161,8 +310,9 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
         int iu, iv, ju, jv;  // tap rows (u) and columns (v) of the chart
         splat_uv(s, p.delta, u, v);
         chart_taps_ij(s, ch, u, v, bilinear, wt, row, fu, fv, iu, iv, ju, jv);
-        // How the texel gradients reach HBM (wave-uniform choice):
-        //   single  1x1 chart, C <= 4: C values in the reduction
+        // How the texel gradients reach HBM (wave-uniform choice; with more
+        // than four channels in texel_gradients_wide):
+        //   single  1x1 chart: C values in the reduction
         //   quad    every valid lane samples the same texel quad, C <= 3:
         //           4 taps x C values in the reduction
         //   window  bilinear, C <= 4, every valid lane's taps inside one 3x3
@@ -172,9 +322,9 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
         //   direct  one atomic per tap
         const int first = __ffsll((unsigned long long)vmask) - 1;
         const int hw = ch.ok ? s.h * s.w : 0;
-        const bool tex_single = hw == 1 && C >= 1 && C <= 4;
+        const bool tex_single = CM <= 4 && hw == 1;
         const int row0 = __builtin_amdgcn_readlane(row[0], first);
-        const bool quad32 = ch.ok && !tex_single && C >= 1 && C <= 3 &&
+        const bool quad32 = CM <= 3 && ch.ok && !tex_single &&
                             !(lanes_where(row[0] != row0) & vmask);
         // window origin (ou, ov): the anchor lane's tap row / column, one
         // lower when some valid lane lies below it (formed only where the
@@ -188,7 +338,7 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
             ov = av - ((lanes_where(iv < av) & vmask) ? 1 : 0);
             win3 = !(lanes_where(((uint32_t)(iu - ou) | (uint32_t)(iv - ov)) > 1u) & vmask);
         }
-        const bool tex_lds = ch.ok && !tex_single && !quad32 && !win3 && C > 0 &&
+        const bool tex_lds = CM <= 4 && ch.ok && !tex_single && !quad32 && !win3 && C > 0 &&
                              hw * C <= kTexAccFloats;
         float* const vtex_chart = b.v_texture + (size_t)(ch.ok ? s.start : 0) * C;
 
@@ -196,7 +346,7 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
         // in the general kernels) and the texel terms of the routes.
         constexpr int NB = G_EXTRA + (GENERAL ? 2 : 0);
         float gr[NB];
-        float vval[CM];  // vis * dL/dtexture_out per channel
+        float vval[CM <= 4 ? CM : 1];  // vis * dL/dtexture_out per channel
         {
             gr[G_RGB + 0] = vis * vo.x;
             gr[G_RGB + 1] = vis * vo.y;
@@ -210,35 +360,17 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
             // differences of two D: coincident taps (equal texels) give equal
             // D and exactly zero.
             float D[4] = {0.f, 0.f, 0.f, 0.f};
-            // texels in chunks of up to 4 channels, all taps loaded before use
-            constexpr int CK = CM < 4 ? CM : 4;
+            if constexpr (CM <= 4) {
+                float tv[4][CM];  // all taps loaded before use
 #pragma unroll
-            for (int cb = 0; cb < CM; cb += CK) {
-                if (cb >= C) break;
-                float tv[4][CK];
+                for (int k = 0; k < 4; ++k)
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
+                    for (int c = 0; c < CM; ++c) tv[k][c] = chart_texel<TB>(ch, row[k] + c * E);
 #pragma unroll
-                    for (int cc = 0; cc < CK; ++cc)
-                        tv[k][cc] = cb + cc < C ? chart_texel<TB>(ch, row[k] + (cb + cc) * E)
-                                                : 0.f;
-                }
+                for (int c = 0; c < CM; ++c) {
 #pragma unroll
-                for (int cc = 0; cc < CK; ++cc) {
-                    const int c = cb + cc;
-                    if (c >= C) break;
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) D[k] = fmaf(tv[k][cc], vtex[c], D[k]);
+                    for (int k = 0; k < 4; ++k) D[k] = fmaf(tv[k][c], vtex[c], D[k]);
                     vval[c] = vis * vtex[c];
-                    if constexpr (CM > 4) {
-                        if (tex_lds) {
-#pragma unroll
-                            for (int k = 0; k < 4; ++k) {
-                                const float add = wt[k] * vval[c];
-                                if (add != 0.f) atomicAdd(acc + (row[k] >> kES) + c, add);
-                            }
-                        }
-                    }
                     if (!tex_single && !quad32 && !win3 && !tex_lds && ch.ok) {
 #pragma unroll
                         for (int k = 0; k < 4; ++k) {
@@ -246,6 +378,30 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
                             if (add != 0.f) unsafeAtomicAdd(vtex_chart + (row[k] >> kES) + c, add);
                         }
                     }
+                }
+            } else {
+                // groups of four channels, a full group's taps in wide loads
+                for (int cb = 0; cb < C; cb += 4) {
+                    float v[4], tv[4][4];
+                    cotangents4(cot, C, cb, v);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        if (cb + 4 <= C) {
+#pragma unroll
+                            for (int c = 0; c < 4; ++c)
+                                tv[k][c] = chart_texel<TB>(ch, row[k] + (cb + c) * E);
+                        } else {
+#pragma unroll
+                            for (int c = 0; c < 4; ++c)
+                                tv[k][c] = cb + c < C
+                                               ? chart_texel<TB>(ch, row[k] + (cb + c) * E)
+                                               : 0.f;
+                        }
+                    }
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) D[k] = fmaf(tv[k][c], v[c], D[k]);
                 }
             }
             vvis += (wt[0] * D[0] + wt[1] * D[1]) + (wt[2] * D[2] + wt[3] * D[3]);
@@ -368,16 +524,17 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
                 if constexpr (CM <= 3) {
                     if (!(lanes_where(rj == 2) & vmask)) {
                         window_texel_add<2, 3, CM>(A, Bw, vval, lane, vtex_chart, ou, ov, s.h,
-                                                   s.w);
+                                                   s.w, CM, CM);
                         return;
                     }
                     if (!(lanes_where(cj == 2) & vmask)) {
                         window_texel_add<3, 2, CM>(A, Bw, vval, lane, vtex_chart, ou, ov, s.h,
-                                                   s.w);
+                                                   s.w, CM, CM);
                         return;
                     }
                 }
-                window_texel_add<3, 3, CM>(A, Bw, vval, lane, vtex_chart, ou, ov, s.h, s.w);
+                window_texel_add<3, 3, CM>(A, Bw, vval, lane, vtex_chart, ou, ov, s.h, s.w, CM,
+                                            CM);
                 return;
             }
             if (tex_lds) {
@@ -397,6 +554,17 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
                         if (q[k] != 0.f) atomicAdd(acc + lofs[k] + c, q[k]);
                 }
             }
+        }
+        if constexpr (CM > 4) {
+            if (ch.ok) {
+                int lofs[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) lofs[k] = row[k] >> kES;
+                texel_gradients_wide(
+                    cot, C, vis, wt, lofs, fu, fv, iu, iv, ju, jv, bilinear, valid, vmask, hw, s.h, s.w,
+                    lane, acc, vtex_chart);
+            }
+            return;
         }
         if (tex_lds) {
             // Flush only the texel rows some valid lane touched.
@@ -482,10 +650,11 @@ __device__ __forceinline__ float* zeroed_tex_acc(float (&tex_acc)[256 / kWave][k
     return acc;
 }
 
-// The plain kernels for CM <= 4 are held to 5 waves per SIMD.
+constexpr int bwd_waves_per_eu(int cm, int mode) { return cm > 4 ? 4 : mode == 0 ? 5 : 1; }
+
 template <int CM, int MODE, bool TB>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(MODE == 0 && CM <= 4 ? 5 : 1)))
+__attribute__((amdgpu_waves_per_eu(bwd_waves_per_eu(CM, MODE))))
 void k_raster_backward(RasterArgs a, BwdIn b) {
     __shared__ float tex_acc[256 / kWave][kTexAccFloats];
     float* const acc = zeroed_tex_acc(tex_acc);
@@ -496,7 +665,7 @@ void k_raster_backward(RasterArgs a, BwdIn b) {
 // forward pass left in `items` (longest list first).
 template <int CM, int MODE, bool TB>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(MODE == 0 && CM <= 4 ? 5 : 1)))
+__attribute__((amdgpu_waves_per_eu(bwd_waves_per_eu(CM, MODE))))
 void k_raster_backward_queue(const ViewRaster* __restrict__ views, ViewsHeader* __restrict__ hdr,
                              const int* __restrict__ items) {
     __shared__ float tex_acc[256 / kWave][kTexAccFloats];
@@ -773,9 +942,7 @@ hipError_t raster_backward_views(const ViewRaster* views, ViewsHeader* hdr, cons
     if (channels == 2) return launch_bwd_queue_cm<2>(views, hdr, items, mode, bf16, blocks, s);
     if (channels == 3) return launch_bwd_queue_cm<3>(views, hdr, items, mode, bf16, blocks, s);
     if (channels == 4) return launch_bwd_queue_cm<4>(views, hdr, items, mode, bf16, blocks, s);
-    if (channels <= 8) return launch_bwd_queue_cm<8>(views, hdr, items, mode, bf16, blocks, s);
-    if (channels <= 16) return launch_bwd_queue_cm<16>(views, hdr, items, mode, bf16, blocks, s);
-    return launch_bwd_queue_cm<64>(views, hdr, items, mode, bf16, blocks, s);
+    return launch_bwd_queue_cm<kRuntimeCM>(views, hdr, items, mode, bf16, blocks, s);
 }
 
 size_t raster_backward_workspace_bytes(int n) {
@@ -802,9 +969,7 @@ hipError_t raster_backward_stage(const RasterCall& c, const float* records,
     if (c.channels == 2) return launch_bwd_cm<2>(a, b, s);
     if (c.channels == 3) return launch_bwd_cm<3>(a, b, s);
     if (c.channels == 4) return launch_bwd_cm<4>(a, b, s);
-    if (c.channels <= 8) return launch_bwd_cm<8>(a, b, s);
-    if (c.channels <= 16) return launch_bwd_cm<16>(a, b, s);
-    return launch_bwd_cm<64>(a, b, s);
+    return launch_bwd_cm<kRuntimeCM>(a, b, s);
 }
 
 hipError_t grad_finalize(int n, const float* grad_rec, const float* records, const float* quats,
