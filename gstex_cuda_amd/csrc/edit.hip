@@ -75,7 +75,7 @@ __global__ __launch_bounds__(256) void k_texture_edit(RasterArgs a, EditIn ed) {
                 rect = wave_rect(!done, j, i);
             }
         }
-        const Window w = window_candidates(a, base, r0, r1 - 1, rect, lane, cull);
+        const Window w = window_candidates<BLUR>(a, base, r0, r1 - 1, rect, lane, cull);
         uint64_t cand = w.cand;
         while (cand != 0) {
             if (!__any(!done)) break;
@@ -250,11 +250,7 @@ hipError_t texture_edit(const RasterCall& c, const float* upd_img, const float* 
     if (e != hipSuccess) return e;
     float* records = (float*)ws;
     if ((e = build_raster_records(c, records, s)) != hipSuccess) return e;
-    RasterArgs a = make_raster_args(c, records);
-    if (c.settings & 1) {  // the edit kernel's blur flag: the box covers the blur disc
-        a.ellipses = nullptr;
-        a.ellipse_c = nullptr;
-    }
+    const RasterArgs a = make_raster_args(c, records);
     const int tiles = a.tiles_x * a.tiles_y;
     if (tiles <= 0) return hipSuccess;
     const EditIn ed{upd_img, upd_alpha, depth_lower, depth_upper, out};

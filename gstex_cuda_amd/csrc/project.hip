@@ -251,8 +251,9 @@ __device__ uint2 cull_box(V3 m, V3 a1, V3 a2, V3 a3, float s1, float s2, float o
                       pack_i16((int)floorf(vmin) - 2, (int)ceilf(vmax) + 2));
 }
 
-// Screen ellipse holding every pixel whose ray can pass the alpha test (blur
-// off), for a per-wave test tighter than the box.  On the splat plane that
+// Screen ellipse holding every pixel whose ray can pass the alpha test by the
+// Gaussian (the blur's disc is tested apart), for a per-wave test tighter than
+// the box.  On the splat plane that
 // region is the ellipse (l1 / (r s1))^2 + (l2 / (r s2))^2 <= 1 with r as in
 // cull_box.  Plane coordinates (l1, l2, 1) map to homogeneous pixel
 // coordinates by G = K Rinv [a1 a2 m-o] (the raster's ray model: pixel

@@ -617,7 +617,7 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
                 // the word again, through the scalar path: no vector register
                 // holds it while the entries are processed
                 const int base = mentry0 + ((wt - k) << 6);
-                const Window w = window_candidates(a, base, r0, e_hi, rect, lane, false);
+                const Window w = window_candidates<false>(a, base, r0, e_hi, rect, lane, false);
                 uint64_t m = mplane_s[wt - k] & w.in_range;
                 while (m != 0) {
                     const int bit = 63 - __builtin_clzll(m);
@@ -630,7 +630,8 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
         return;
     }
     for (int base = e_hi >= r0 ? (e_hi & ~63) : mentry0 - 64; base >= mentry0; base -= 64) {
-        const Window w = window_candidates(a, base, r0, e_hi, rect, lane, a.boxes != nullptr);
+        const Window w = window_candidates<GENERAL>(a, base, r0, e_hi, rect, lane,
+                                                    a.boxes != nullptr, use_blur);
         uint64_t m = w.cand;
         while (m != 0) {
             const int bit = 63 - __builtin_clzll(m);
