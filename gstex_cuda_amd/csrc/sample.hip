@@ -26,22 +26,41 @@ __device__ __forceinline__ void sample_taps(int h, int w, int start, float u, fl
     row[3] = min(max(start + ju * w + jv, 0), lim);
 }
 
-__global__ __launch_bounds__(256) void k_sample_forward(int q, int C, int num_texels,
+// One thread per query.  CM is the channel count, or 0 for a runtime count: the
+// exact counts read a tap as one wide load, so a query makes 4 gathers instead
+// of 4 C (each gather instruction of a wave touches up to 64 cache lines, which
+// is what bounds this kernel).  4M queries of 3 channels over 2M texels:
+// 135 us with a gather per value, 93 with one per tap.
+template <int CM>
+__global__ __launch_bounds__(256) void k_sample_forward(int q, int channels, int num_texels,
                                                         const int* __restrict__ dims,
                                                         const float* __restrict__ uvs,
                                                         const float* __restrict__ texture,
                                                         float* __restrict__ out) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= q) return;
+    const int C = CM ? CM : channels;
     float wt[4];
     int row[4];
     sample_taps(dims[3 * i], dims[3 * i + 1], dims[3 * i + 2], uvs[2 * i], uvs[2 * i + 1],
                 num_texels, wt, row);
-    for (int c = 0; c < C; ++c)
-        out[(size_t)i * C + c] = wt[0] * texture[(size_t)row[0] * C + c] +
-                                 wt[1] * texture[(size_t)row[1] * C + c] +
-                                 wt[2] * texture[(size_t)row[2] * C + c] +
-                                 wt[3] * texture[(size_t)row[3] * C + c];
+    if constexpr (CM != 0) {
+        float t[4][CM];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int c = 0; c < CM; ++c) t[k][c] = texture[(size_t)row[k] * CM + c];
+#pragma unroll
+        for (int c = 0; c < CM; ++c)
+            out[(size_t)i * CM + c] =
+                wt[0] * t[0][c] + wt[1] * t[1][c] + wt[2] * t[2][c] + wt[3] * t[3][c];
+    } else {
+        for (int c = 0; c < C; ++c)
+            out[(size_t)i * C + c] = wt[0] * texture[(size_t)row[0] * C + c] +
+                                     wt[1] * texture[(size_t)row[1] * C + c] +
+                                     wt[2] * texture[(size_t)row[2] * C + c] +
+                                     wt[3] * texture[(size_t)row[3] * C + c];
+    }
 }
 
 // Taps that clamp onto one texel (every tap of a 1x1 chart, the far edge of
@@ -104,13 +123,48 @@ constexpr int kSamplePer = 16;
 constexpr int kSampleRange = 256 * kSamplePer;
 constexpr int kSampleWindow = 8192;  // floats (32 KiB)
 
+// One query's adds: the taps of channel value g(c) into the window or HBM.
+template <int CM, typename G>
+__device__ __forceinline__ void sample_scatter(int C, int num_texels, int h, int w, int start,
+                                               float u, float v, const G& g, long long base,
+                                               float* win, float* v_texture, int& hi) {
+    float wt[4];
+    int row[4];
+    sample_taps(h, w, start, u, v, num_texels, wt, row);
+    merge_taps(wt, row);
+#pragma unroll
+    for (int c = 0; c < (CM ? CM : C); ++c) {
+        const float gc = g(c);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const float add = wt[t] * gc;
+            if (add == 0.f) continue;
+            const long long at = (long long)row[t] * C + c;
+            const long long off = at - base;
+            if (off >= 0 && off < kSampleWindow) {
+                atomicAdd(win + off, add);
+                hi = max(hi, (int)off + 1);
+            } else {
+                unsafeAtomicAdd(v_texture + at, add);
+            }
+        }
+    }
+}
+
+// CM 1..4: that many channels, through the packed records; 0: a runtime count,
+// from the original arrays.  With records a thread takes its queries four at a
+// time, the four gathers in flight together, and the exact count keeps the
+// cotangents in registers (an index at run time put them in scratch memory):
+// 4M queries of 3 channels, 141 -> 117 us.
+template <int CM>
 __global__ __launch_bounds__(256) void k_sample_backward_sorted(
-    int q, int C, int num_texels, const uint32_t* __restrict__ keys_sorted,
+    int q, int channels, int num_texels, const uint32_t* __restrict__ keys_sorted,
     const uint32_t* __restrict__ idx_sorted, const float4* __restrict__ rec,
     const int* __restrict__ dims, const float* __restrict__ uvs, const float* __restrict__ v_out,
     float* __restrict__ v_texture) {
     __shared__ float win[kSampleWindow];
     __shared__ int used;
+    const int C = CM ? CM : channels;
     const int first = blockIdx.x * kSampleRange;
     const int last = min(first + kSampleRange, q);
     for (int k = threadIdx.x; k < kSampleWindow; k += blockDim.x) win[k] = 0.f;
@@ -118,52 +172,39 @@ __global__ __launch_bounds__(256) void k_sample_backward_sorted(
     __syncthreads();
     const long long base = ((long long)keys_sorted[first] << kSampleBucketShift) * C;
     int hi = 0;  // past the last window value this thread touched
-    const int k0 = first + threadIdx.x * kSamplePer;
-    for (int k = k0; k < min(k0 + kSamplePer, last); ++k) {
-        const int i = (int)idx_sorted[k];
-        int h, w, start;
-        float u, v, g[4];
-        bool packed = false;
-        if (rec != nullptr) {
-            const float4 a = rec[2 * (size_t)i];
-            const float4 b = rec[2 * (size_t)i + 1];
-            const uint32_t hw = __float_as_uint(a.w);
-            packed = hw != kSampleUnpacked;
-            u = a.x;
-            v = a.y;
-            start = __float_as_int(a.z);
-            h = (int)(hw & 0xffffu);
-            w = (int)(hw >> 16);
-            g[0] = b.x;
-            g[1] = b.y;
-            g[2] = b.z;
-            g[3] = b.w;
-        }
-        if (!packed) {
-            h = dims[3 * i];
-            w = dims[3 * i + 1];
-            start = dims[3 * i + 2];
-            u = uvs[2 * i];
-            v = uvs[2 * i + 1];
-        }
-        float wt[4];
-        int row[4];
-        sample_taps(h, w, start, u, v, num_texels, wt, row);
-        merge_taps(wt, row);
-        for (int c = 0; c < C; ++c) {
-            const float gc = packed ? g[c & 3] : v_out[(size_t)i * C + c];
+    const int k0 = first + threadIdx.x * kSamplePer, k1 = min(k0 + kSamplePer, last);
+    auto from_arrays = [&](int i) {
+        const float* g = v_out + (size_t)i * C;
+        sample_scatter<CM>(
+            C, num_texels, dims[3 * i], dims[3 * i + 1], dims[3 * i + 2], uvs[2 * i],
+            uvs[2 * i + 1], [&](int c) { return g[c]; }, base, win, v_texture, hi);
+    };
+    if constexpr (CM == 0) {
+        for (int k = k0; k < k1; ++k) from_arrays((int)idx_sorted[k]);
+    } else {
+        constexpr int kTake = 4;
+        for (int k = k0; k < k1; k += kTake) {
+            int id[kTake];
+            float4 a[kTake], b[kTake];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const float add = wt[t] * gc;
-                if (add == 0.f) continue;
-                const long long at = (long long)row[t] * C + c;
-                const long long off = at - base;
-                if (off >= 0 && off < kSampleWindow) {
-                    atomicAdd(win + off, add);
-                    hi = max(hi, (int)off + 1);
-                } else {
-                    unsafeAtomicAdd(v_texture + at, add);
+            for (int j = 0; j < kTake; ++j) id[j] = (int)idx_sorted[min(k + j, k1 - 1)];
+#pragma unroll
+            for (int j = 0; j < kTake; ++j) {
+                a[j] = rec[2 * (size_t)id[j]];
+                b[j] = rec[2 * (size_t)id[j] + 1];
+            }
+#pragma unroll
+            for (int j = 0; j < kTake; ++j) {
+                if (k + j >= k1) break;
+                const uint32_t hw = __float_as_uint(a[j].w);
+                if (hw == kSampleUnpacked) {
+                    from_arrays(id[j]);
+                    continue;
                 }
+                const float g4[4] = {b[j].x, b[j].y, b[j].z, b[j].w};
+                sample_scatter<CM>(
+                    C, num_texels, (int)(hw & 0xffffu), (int)(hw >> 16), __float_as_int(a[j].z),
+                    a[j].x, a[j].y, [&](int c) { return g4[c]; }, base, win, v_texture, hi);
             }
         }
     }
@@ -179,7 +220,14 @@ __global__ __launch_bounds__(256) void k_sample_backward_sorted(
 hipError_t sample_forward(int q, int C, int num_texels, const int* dims, const float* uvs,
                           const float* texture, float* out, hipStream_t s) {
     if (q <= 0 || C <= 0) return hipSuccess;
-    k_sample_forward<<<(q + 255) / 256, 256, 0, s>>>(q, C, num_texels, dims, uvs, texture, out);
+    const int g = (q + 255) / 256;
+    switch (C) {
+        case 1: k_sample_forward<1><<<g, 256, 0, s>>>(q, C, num_texels, dims, uvs, texture, out); break;
+        case 2: k_sample_forward<2><<<g, 256, 0, s>>>(q, C, num_texels, dims, uvs, texture, out); break;
+        case 3: k_sample_forward<3><<<g, 256, 0, s>>>(q, C, num_texels, dims, uvs, texture, out); break;
+        case 4: k_sample_forward<4><<<g, 256, 0, s>>>(q, C, num_texels, dims, uvs, texture, out); break;
+        default: k_sample_forward<0><<<g, 256, 0, s>>>(q, C, num_texels, dims, uvs, texture, out);
+    }
     return hipGetLastError();
 }
 
@@ -215,8 +263,18 @@ hipError_t sample_backward(int q, int C, int num_texels, const int* dims, const 
     const int end_bit = 32 - __builtin_clz(((unsigned)num_texels >> kSampleBucketShift) | 1u);
     e = sort_u32_pairs(q, keys, idx, keys_s, idx_s, end_bit, rws, rws_bytes, s);
     if (e != hipSuccess) return e;
-    k_sample_backward_sorted<<<(q + kSampleRange - 1) / kSampleRange, 256, 0, s>>>(
-        q, C, num_texels, keys_s, idx_s, rec, dims, uvs, v_out, v_texture);
+    const int g = (q + kSampleRange - 1) / kSampleRange;
+#define GSTEX_SAMPLE_BWD(CM)                                                                  \
+    k_sample_backward_sorted<CM><<<g, 256, 0, s>>>(q, C, num_texels, keys_s, idx_s, rec, dims, \
+                                                   uvs, v_out, v_texture)
+    switch (C) {
+        case 1: GSTEX_SAMPLE_BWD(1); break;
+        case 2: GSTEX_SAMPLE_BWD(2); break;
+        case 3: GSTEX_SAMPLE_BWD(3); break;
+        case 4: GSTEX_SAMPLE_BWD(4); break;
+        default: GSTEX_SAMPLE_BWD(0);
+    }
+#undef GSTEX_SAMPLE_BWD
     return hipGetLastError();
 }
 
