@@ -445,6 +445,7 @@ hipError_t raster_forward_stage(const RasterCall& c, const float* records, float
     const FwdOut o{out_img, out_depth, out_reg, out_texture, out_normal,
                    final_Ts, final_idx, depth_idx, out_reg_s};
     if (a.tiles_x * a.tiles_y <= 0) return hipSuccess;
+    if (raster_forward_is_narrow(a)) return raster_forward_narrow(a, o, s);
     if (c.channels == 1) return launch_fwd_cm<1>(a, o, s);
     if (c.channels == 2) return launch_fwd_cm<2>(a, o, s);
     if (c.channels == 3) return launch_fwd_cm<3>(a, o, s);

@@ -966,6 +966,7 @@ hipError_t raster_backward_stage(const RasterCall& c, const float* records,
     const BwdIn b{final_Ts, final_idx, depth_idx, final_s, v_img, v_depth, v_reg, v_alpha,
                   v_texture_out, v_normal, grad_rec, v_texture, loss_target, loss_scale};
     if (a.tiles_x * a.tiles_y <= 0) return hipSuccess;
+    if (raster_backward_is_narrow(a)) return raster_backward_narrow(a, b, s);
     if (c.channels == 1) return launch_bwd_cm<1>(a, b, s);
     if (c.channels == 2) return launch_bwd_cm<2>(a, b, s);
     if (c.channels == 3) return launch_bwd_cm<3>(a, b, s);

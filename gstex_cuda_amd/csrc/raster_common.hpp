@@ -751,6 +751,25 @@ inline RasterArgs make_raster_args(const RasterCall& c, const float* records) {
     return a;
 }
 
+// The kernels of raster_narrow.hip take grids of up to kNarrowTiles tiles
+// whose lists hold at most kNarrowForwardIds (kNarrowBackwardIds) entries:
+// there the 8x8 kernels are bound by their longest wave.  With more work the
+// chip fills, and the narrow kernels' instruction count, about twice that of
+// the 8x8 kernels on full waves, decides.  Measured (forward + backward of
+// three channels, 8x8 against narrow): 256 tiles, 66K entries 263 + 431 us
+// against 114 + 193; 920 tiles, 96K 223 + 368 against 112 + 208; 920 tiles,
+// 480K 199 + 383 against 133 + 327; 900 tiles, 405K 186 + 336 against
+// 140 + 335; 1350 tiles, 271K 175 + 303 against 133 + 294; but 1024 tiles,
+// 737K 177 + 375 against 175 + 436, 1900 tiles, 120K 101 + 209 against
+// 113 + 232 and 3600 tiles, 97K 76 + 160 against 113 + 229.
+constexpr int kNarrowTiles = 1400;
+constexpr int kNarrowForwardIds = 600000;
+constexpr int kNarrowBackwardIds = 450000;
+bool raster_forward_is_narrow(const RasterArgs& a);
+bool raster_backward_is_narrow(const RasterArgs& a);
+hipError_t raster_forward_narrow(const RasterArgs& a, const FwdOut& o, hipStream_t s);
+hipError_t raster_backward_narrow(const RasterArgs& a, const BwdIn& b, hipStream_t s);
+
 inline hipError_t build_raster_records(const RasterCall& c, float* records, hipStream_t s) {
     return launch_build_records(c.num_points, c.means, c.scales, c.glob_scale, c.quats, c.colors,
                                 c.opacities, c.uv0, c.umap, c.vmap, c.texture_dims, c.viewmat,
