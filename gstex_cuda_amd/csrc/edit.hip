@@ -8,9 +8,17 @@
 // (r*a, g*a, b*a, a, 1) are added to channels 0..4 of the output, a being the
 // pixel's edit alpha.  The walk is the forward's: quadrant waves, 64-entry
 // windows with screen-box culling, SMEM records.  The values reach the output
-// by the texel routes of the raster backward: wave reduce-scatters for one
-// texel, a shared texel quad or a 3x3 texel window, else DPP-merged lanes into
-// an LDS accumulator or direct float atomics.
+// through matrix instructions for a shared texel quad or a window of up to 3x3
+// texels, else by DPP-merged lanes into an LDS accumulator or direct float
+// atomics.
+//
+// Bound by VALU issue (0.8 of the issue slots).  500k Gaussians on a 1080p
+// canvas: 897 us with wave reductions of all taps x 5 values in a branch of the
+// live lanes, 711 with wave masks in the branch's place and 2x3 and 3x2
+// windows, 609 with the matrix instructions (280 of it the walk).  The plain
+// kernels are held to 96 VGPRs, five waves per SIMD (four: 748 against 711).
+#include <type_traits>
+
 #include "raster_common.hpp"
 
 namespace gstex {
@@ -23,8 +31,39 @@ struct EditIn {
     float* out;                // (X, C), C >= 5
 };
 
-template <bool BLUR>
-__global__ __launch_bounds__(256) void k_texture_edit(RasterArgs a, EditIn ed) {
+// Adds to the texels of one window the sums over the wave's pixels of weight x
+// (4 channels, 1): rows[r] holds the weights of window row r's texels (of all
+// four texels of a quad, R = 1, Q = 4), value the channels of the pixel quad.
+// at(r, q): the texel's first value.  Channel 4: lane i of a pixel quad sums
+// texel i's weights over the quad.  A zero sum is not added; window rows and
+// columns past the chart carry no weight.
+template <int R, int Q, typename At>
+__device__ __forceinline__ void window_add(const float (&rows)[R][4], const float (&value)[4],
+                                           int lane, float* chart, At at) {
+    constexpr int N = R * Q;
+    float v[N + R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        quad_sums<Q>(rows[r], value, v + Q * r);
+        v[N + r] = (rows[r][0] + rows[r][1]) + (rows[r][2] + rows[r][3]);
+    }
+    const float tot = quad_reduce_scatter(v, lane);
+    const int code = quad_slot<N + R>(lane), j = lane & 3;
+    const bool one = code >= N;  // bit 6 (a copy) makes it larger still
+    const int r = one ? code - N : code / Q, q = one ? j : code - Q * (code / Q);
+    if (code < 64 && q < Q && tot != 0.f) unsafeAtomicAdd(chart + at(r, q) + (one ? 4 : j), tot);
+}
+
+// Chart::ok of chart_of (float values).
+__device__ __forceinline__ bool chart_inside(const Splat& s, int C, int num_texels) {
+    const uint32_t h = (uint32_t)s.h, w = (uint32_t)s.w, n = h * w, X = (uint32_t)num_texels;
+    const uint32_t over = __umulhi(h, w) | __umulhi(n, 4u * C) | ((n * 4u * C) >> 31);
+    return (over == 0) & (max(h - 1u, w - 1u) < 0xffffffu) & (n <= X) & ((uint32_t)s.start <= X - n);
+}
+
+template <bool BLUR, bool PRECISE>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(PRECISE ? 1 : 5))) void k_texture_edit(RasterArgs a, EditIn ed) {
     const int tile = blockIdx.x;
     const int ty = tile / a.tiles_x, tx = tile - ty * a.tiles_x;
     const int lane = threadIdx.x & (kWave - 1);
@@ -49,193 +88,194 @@ __global__ __launch_bounds__(256) void k_texture_edit(RasterArgs a, EditIn ed) {
     }
     int r0, r1;
     tile_range(a, tile, r0, r1);
-    bool done = !inside;
     float T = 1.f;
     // culling rectangle of the live pixels (shrinks as pixels finish, as in
     // k_raster_forward)
     WaveRect rect = wave_rect(inside, j, i);
-    int live = __popcll(__ballot(inside));
+    uint64_t live = lanes_where(inside);  // pixels still compositing
+    int live_n = __popcll(live);
     // wave-private texel accumulator, kept zero between Gaussians by the flush
     __shared__ float tex_acc[256 / kWave][kTexAccFloats];
     float* acc = tex_acc[wave_index()];
     for (int k = lane; k < kTexAccFloats; k += kWave) acc[k] = 0.f;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    const float inv_c4 = 1.f / (float)(4 * C);  // chart byte offset -> texel index
     // a pixel with T (1 - 1/255) <= 1e-4 can take no further entry (each one
     // with alpha >= 1/255 ends it), so it stops at once and culled entries
     // never matter (as in k_raster_forward)
     constexpr float kKeep = 1.f - 1.f / 255.f;
     const bool cull = a.boxes != nullptr;
-    for (int base = r0 & ~63; base < r1; base += 64) {
-        if (!__any(!done)) break;
-        {
-            const int now = __popcll(__ballot(!done));
-            if (now < live) {
-                live = now;
-                rect = wave_rect(!done, j, i);
+
+    // products with the zero weights of other pixels' texels need finite values
+    const bool finite = lanes_where(!(fabsf(val[0]) < INFINITY && fabsf(val[1]) < INFINITY &&
+                                      fabsf(val[2]) < INFINITY && fabsf(val[3]) < INFINITY)) == 0;
+    // channels 0..3 of the pixels of this lane's quad, channel lane & 3
+    float quad_val[4];
+    {
+        const int c = lane & 3;
+        auto pick = [&](float v0, float v1, float v2, float v3) {
+            return c == 0 ? v0 : c == 1 ? v1 : c == 2 ? v2 : v3;
+        };
+#define GSTEX_QUAD_VAL(M)                                                                       \
+    quad_val[M] = pick(quad_lane<M>(val[0]), quad_lane<M>(val[1]), quad_lane<M>(val[2]),        \
+                       quad_lane<M>(val[3]))
+        GSTEX_QUAD_VAL(0);
+        GSTEX_QUAD_VAL(1);
+        GSTEX_QUAD_VAL(2);
+        GSTEX_QUAD_VAL(3);
+#undef GSTEX_QUAD_VAL
+    }
+
+    // One list entry: Gaussian g with record s.  The pair math runs for every
+    // lane (finite for any pixel ray); the live, composited and hitting pixels
+    // are wave masks.
+    auto entry = [&](const Splat& s) {
+        const Pair p = pair_eval(s, pr, BLUR, PRECISE);
+        const float next_T = T * (1.f - p.alpha);
+        live &= ~lanes_where(next_T <= 1e-4f);
+        const uint64_t comp = live & ~skip_lanes(p);
+        if (comp == 0) return;
+        const float t_view = p.t * pr.view_depth;
+        const uint64_t hm = comp & lanes_where(t_view >= lo) & lanes_where(t_view <= hi);
+        const bool composited = __builtin_amdgcn_inverse_ballot_w64(comp);
+        T = composited ? next_T : T;
+        live &= ~(comp & lanes_where(next_T * kKeep <= 1e-4f));
+        // out has the texture's (X, C) float layout; charts outside it get nothing
+        if (hm == 0 || !chart_inside(s, C, a.num_texels)) return;
+        const bool hit = __builtin_amdgcn_inverse_ballot_w64(hm);
+        float* const out_chart = ed.out + (size_t)s.start * C;
+        const int first = __ffsll((unsigned long long)hm) - 1;
+        // How the (taps x 5) values reach the output (wave-uniform choice):
+        //   quad    every hitting lane samples one texel quad (a 1x1 chart too),
+        //   window  or its taps lie inside one 2x3, 3x2 or 3x3 texel window:
+        //           matrix instructions (window_add), one atomic per texel
+        //           and value
+        //   lds     charts of up to kTexAccFloats / 5 texels: merged lanes
+        //           add into the wave's LDS accumulator, then flush
+        //   direct  one atomic per tap and value (all entries of a wave with
+        //           a value that is not finite: only its own texels take it)
+        auto quad = [&](float y, float x, int ou, int ov) {
+            QuadWeights qw;
+            qw.set(y, x, hit ? 1.f : 0.f, lane);
+            const float rows[1][4] = {{qw.w[0], qw.w[1], qw.w[2], qw.w[3]}};
+            const int o = ou * s.w + ov;
+            window_add<1, 4>(rows, quad_val, lane, out_chart,
+                             [&](int, int q) { return (o + (q & 1) + (q >> 1) * s.w) * C; });
+        };
+        if (s.h * s.w == 1 && finite) {
+            quad(0.f, 0.f, 0, 0);
+            return;
+        }
+        // position in texels, with replicate padding: past the last texel's
+        // centre both taps are that texel, as at its centre
+        float u, v;
+        splat_uv(s, p.delta, u, v);
+        const float tu = fminf((float)s.h * u, (float)(s.h - 1));
+        const float tv = fminf((float)s.w * v, (float)(s.w - 1));
+        const float flu = floorf(tu), flv = floorf(tv);
+        // position relative to the first hitting lane's taps
+        const float au = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(flu), first));
+        const float av = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(flv), first));
+        const float y0 = tu - au, x0 = tv - av;
+        const int iu0 = (int)au, iv0 = (int)av;
+        auto outside = [&](float t, float top) {
+            return lanes_where(fminf(fmaxf(t, 0.f), top) != t) & hm;
+        };
+        const bool ou1 = outside(y0, 1.f) != 0, ov1 = outside(x0, 1.f) != 0;
+        if (finite && !ou1 && !ov1) {
+            quad(y0, x0, iu0, iv0);
+            return;
+        }
+        // window origin: one texel lower where some hitting lane lies below
+        const bool lu = (lanes_where(y0 < 0.f) & hm) != 0, lv = (lanes_where(x0 < 0.f) & hm) != 0;
+        const float y = y0 + (lu ? 1.f : 0.f), x = x0 + (lv ? 1.f : 0.f);
+        if (finite && !(outside(y, 2.f) | outside(x, 2.f))) {
+            const int o = (iu0 - (lu ? 1 : 0)) * s.w + iv0 - (lv ? 1 : 0);
+            auto at = [&](int r, int q) { return (o + r * s.w + q) * C; };
+            // a pixel that does not hit has no column weights
+            const float xh = hit ? x : 8.f;
+            auto window = [&](auto R, auto Q) {
+                float a[R.value];
+                row_weights(y, a);
+                WindowWeights<R.value> ww;
+                ww.set(a, xh, lane);
+                window_add<R.value, Q.value>(ww.w, quad_val, lane, out_chart, at);
+            };
+            using two = std::integral_constant<int, 2>;
+            using three = std::integral_constant<int, 3>;
+            if (!outside(y, 1.f)) window(two{}, three{});
+            else if (!outside(x, 1.f)) window(three{}, two{});
+            else window(three{}, three{});
+            return;
+        }
+        const int iu = (int)flu, iv = (int)flv;  // tap rows and columns
+        const int ju = min(iu + 1, s.h - 1), jv = min(iv + 1, s.w - 1);
+        const float fu = tu - flu, fv = tv - flv;
+        const float a0 = hit ? 1.f - fu : 0.f, a1 = hit ? fu : 0.f;
+        const float wt[4] = {a0 * (1.f - fv), a0 * fv, a1 * (1.f - fv), a1 * fv};
+        const int tix[4] = {iu * s.w + iv, iu * s.w + jv, ju * s.w + iv, ju * s.w + jv};
+        if (!finite) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int k = 0; k < 5; ++k)
+                    if (wt[t] != 0.f)
+                        unsafeAtomicAdd(out_chart + (size_t)tix[t] * C + k, wt[t] * val[k]);
+            return;
+        }
+        const QuadMerge qm = quad_merge_setup(hit ? tix[0] : -1, lane);
+        if (s.h * s.w * 5 <= kTexAccFloats) {
+            // charts of up to kTexAccFloats / 5 texels: merged lanes add into
+            // the wave's LDS accumulator (5 values per texel), then the texels
+            // some lane touched go out with one atomic each
+#pragma unroll
+            for (int k = 0; k < 5; ++k) {
+                float q[4];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) q[t] = quad_merge(wt[t] * val[k], qm);
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    if (q[t] != 0.f) atomicAdd(acc + tix[t] * 5 + k, q[t]);
             }
+            // tap 0 is the lowest texel of a lane's quad, tap 3 the highest
+            const int tlo = wave_min(hit ? tix[0] : 0x7fffffff);
+            const int thi = wave_max(hit ? tix[3] : -1);
+            // every lane's LDS adds precede these reads in the wave's LDS queue
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            const int nv = (thi - tlo + 1) * 5;
+            for (int idx = lane; idx < nv; idx += kWave) {
+                const int tx = tlo + idx / 5, k = idx - (idx / 5) * 5;
+                const float v = acc[tx * 5 + k];
+                if (v != 0.f) {
+                    unsafeAtomicAdd(out_chart + (size_t)tx * C + k, v);
+                    acc[tx * 5 + k] = 0.f;
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            return;
+        }
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+            float q[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) q[t] = quad_merge(wt[t] * val[k], qm);
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                if (q[t] != 0.f) unsafeAtomicAdd(out_chart + (size_t)tix[t] * C + k, q[t]);
+        }
+    };
+
+    for (int base = r0 & ~63; base < r1 && live != 0; base += 64) {
+        const int now = __popcll(live);
+        if (now < live_n) {
+            live_n = now;
+            rect = wave_rect(__builtin_amdgcn_inverse_ballot_w64(live), j, i);
         }
         const Window w = window_candidates<BLUR>(a, base, r0, r1 - 1, rect, lane, cull);
         uint64_t cand = w.cand;
-        while (cand != 0) {
-            if (!__any(!done)) break;
+        while (cand != 0 && live != 0) {
             const int bit = __ffsll((unsigned long long)cand) - 1;
             cand &= cand - 1;
-            const int g = __builtin_amdgcn_readlane(w.gid, bit);
-            const Splat s = splat_record(a, g);
-            bool hit = false;
-            float wt[4] = {0.f, 0.f, 0.f, 0.f};
-            int row[4] = {0, 0, 0, 0};  // byte offsets inside the chart (float values)
-            float fu = 0.f, fv = 0.f;
-            int iu = 0, iv = 0, ju = 0, jv = 0;  // tap rows (u) and columns (v)
-            // out has the texture's (X, C) float layout; charts outside it get nothing
-            const Chart ch = chart_of<false>(ed.out, s, C, a.num_texels);
-            if (!done) {
-                const Pair p = pair_eval(s, pr, BLUR, a.precise_edge);
-                const float next_T = T * (1.f - p.alpha);
-                if (next_T <= 1e-4f) done = true;
-                if (!(p.skip || done)) {
-                    const float t_view = p.t * pr.view_depth;
-                    if (t_view >= lo && t_view <= hi) {
-                        hit = true;
-                        float u, v;
-                        splat_uv(s, p.delta, u, v);
-                        chart_taps_ij(s, ch, u, v, true, wt, row, fu, fv, iu, iv, ju, jv);
-                    }
-                    T = next_T;
-                    if (T * kKeep <= 1e-4f) done = true;
-                }
-            }
-            if (!__any(hit) || !ch.ok) continue;
-            float* const out_chart = ed.out + (size_t)s.start * C;
-            // How the (taps x 5) values reach the output (wave-uniform choice,
-            // as for the texel gradients of the raster backward):
-            //   single  1x1 chart: 5 values in a wave reduce-scatter
-            //   quad    every hitting lane samples the same texel quad: 20 values
-            //   window  every hitting lane's taps lie in one 3x3 texel window:
-            //           the 9 separable weight products x 5 values
-            //   lds     charts of up to kTexAccFloats / 5 texels: merged lanes
-            //           add into the wave's LDS accumulator, then flush
-            //   direct  one atomic per tap and value
-            // Lanes that do not hit have zero weights, so they add nothing.
-            const int first = __ffsll((unsigned long long)__ballot(hit)) - 1;
-            if (s.h * s.w == 1) {
-                const float ws = (wt[0] + wt[1]) + (wt[2] + wt[3]);
-                float v5[5];
-#pragma unroll
-                for (int k = 0; k < 5; ++k) v5[k] = ws * val[k];
-                const float tot = wave_reduce_scatter(v5, lane);
-                const int code = rs_slot<5>(lane);
-                if (code < 64 && tot != 0.f) unsafeAtomicAdd(out_chart + code, tot);
-                continue;
-            }
-            const int row0 = __builtin_amdgcn_readlane(row[0], first);
-            if (!__any(hit && row[0] != row0)) {
-                const int row1 = __builtin_amdgcn_readlane(row[1], first);
-                const int row2 = __builtin_amdgcn_readlane(row[2], first);
-                const int row3 = __builtin_amdgcn_readlane(row[3], first);
-                float v20[20];
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-#pragma unroll
-                    for (int k = 0; k < 5; ++k) v20[5 * t + k] = wt[t] * val[k];
-                const float tot = wave_reduce_scatter(v20, lane);
-                const int code = rs_slot<20>(lane);
-                if (code < 64 && tot != 0.f) {
-                    const int t = code / 5, k = code - 5 * t;
-                    const int rr = t == 0 ? row0 : t == 1 ? row1 : t == 2 ? row2 : row3;
-                    unsafeAtomicAdd(out_chart + (rr >> 2) + k, tot);
-                }
-                continue;
-            }
-            {
-                // window origin: the first hitting lane's tap row / column, one
-                // lower when some hitting lane lies below it
-                const int au = __builtin_amdgcn_readlane(iu, first);
-                const int av = __builtin_amdgcn_readlane(iv, first);
-                const int ou = au - (__any(hit && iu < au) ? 1 : 0);
-                const int ov = av - (__any(hit && iv < av) ? 1 : 0);
-                if (!__any(hit && (iu < ou || iu > ou + 1 || iv < ov || iv > ov + 1))) {
-                    // tap (row r, column q) has weight A[r] * B[q]; rows iu, ju and
-                    // columns iv, jv relative to the origin lie in 0..2
-                    const float h1 = hit ? 1.f : 0.f;
-                    const float wa0 = h1 * (1.f - fu), wa1 = h1 * fu, wb0 = 1.f - fv, wb1 = fv;
-                    const int ri = iu - ou, rj = ju - ou, ci = iv - ov, cj = jv - ov;
-                    float A[3], Bw[3];
-#pragma unroll
-                    for (int r = 0; r < 3; ++r) {
-                        A[r] = (ri == r ? wa0 : 0.f) + (rj == r ? wa1 : 0.f);
-                        Bw[r] = (ci == r ? wb0 : 0.f) + (cj == r ? wb1 : 0.f);
-                    }
-                    float v45[45];
-#pragma unroll
-                    for (int r = 0; r < 3; ++r)
-#pragma unroll
-                        for (int q = 0; q < 3; ++q) {
-                            const float ab = A[r] * Bw[q];
-#pragma unroll
-                            for (int k = 0; k < 5; ++k) v45[(3 * r + q) * 5 + k] = ab * val[k];
-                        }
-                    const float tot = wave_reduce_scatter(v45, lane);
-                    const int code = rs_slot<45>(lane);
-                    if (code < 64 && tot != 0.f) {
-                        const int rq = code / 5, k = code - 5 * rq;
-                        const int r = rq / 3, q = rq - 3 * r;
-                        // a window row or column past the chart edge has no weight
-                        if (ou + r < s.h && ov + q < s.w)
-                            unsafeAtomicAdd(out_chart + ((size_t)(ou + r) * s.w + (ov + q)) * C + k,
-                                            tot);
-                    }
-                    continue;
-                }
-            }
-            const QuadMerge qm = quad_merge_setup(hit ? row[0] : -1, lane);
-            if (s.h * s.w * 5 <= kTexAccFloats) {
-                // charts of up to kTexAccFloats / 5 texels: merged lanes add
-                // into the wave's LDS accumulator (5 values per texel), then
-                // the texels some lane touched go out with one atomic each
-                int tix[4];
-#pragma unroll
-                for (int t = 0; t < 4; ++t) tix[t] = (int)((float)row[t] * inv_c4 + 0.5f);
-#pragma unroll
-                for (int k = 0; k < 5; ++k) {
-                    float q[4];
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) q[t] = quad_merge(wt[t] * val[k], qm);
-#pragma unroll
-                    for (int t = 0; t < 4; ++t)
-                        if (q[t] != 0.f) atomicAdd(acc + tix[t] * 5 + k, q[t]);
-                }
-                int tlo = 0x7fffffff, thi = -1;
-                if (hit) {
-                    tlo = min(min(tix[0], tix[1]), min(tix[2], tix[3]));
-                    thi = max(max(tix[0], tix[1]), max(tix[2], tix[3]));
-                }
-                tlo = wave_min(tlo);
-                thi = wave_max(thi);
-                // every lane's LDS adds precede these reads in the wave's LDS queue
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                const int nv = (thi - tlo + 1) * 5;
-                for (int idx = lane; idx < nv; idx += kWave) {
-                    const int tx = tlo + idx / 5, k = idx - (idx / 5) * 5;
-                    const float v = acc[tx * 5 + k];
-                    if (v != 0.f) {
-                        unsafeAtomicAdd(out_chart + (size_t)tx * C + k, v);
-                        acc[tx * 5 + k] = 0.f;
-                    }
-                }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            } else {
-#pragma unroll
-                for (int k = 0; k < 5; ++k) {
-                    float q[4];
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) q[t] = quad_merge(wt[t] * val[k], qm);
-#pragma unroll
-                    for (int t = 0; t < 4; ++t)
-                        if (q[t] != 0.f) unsafeAtomicAdd(out_chart + (row[t] >> 2) + k, q[t]);
-                }
-            }
+            entry(splat_record(a, __builtin_amdgcn_readlane(w.gid, bit)));
         }
     }
 }
@@ -254,10 +294,12 @@ hipError_t texture_edit(const RasterCall& c, const float* upd_img, const float* 
     const int tiles = a.tiles_x * a.tiles_y;
     if (tiles <= 0) return hipSuccess;
     const EditIn ed{upd_img, upd_alpha, depth_lower, depth_upper, out};
-    if (c.settings & 1)
-        k_texture_edit<true><<<tiles, raster_block_threads(a.bw), 0, s>>>(a, ed);
-    else
-        k_texture_edit<false><<<tiles, raster_block_threads(a.bw), 0, s>>>(a, ed);
+    const dim3 block(raster_block_threads(a.bw));
+    auto* const kernel = c.settings & 1 ? (a.precise_edge ? k_texture_edit<true, true>
+                                                          : k_texture_edit<true, false>)
+                                        : (a.precise_edge ? k_texture_edit<false, true>
+                                                          : k_texture_edit<false, false>);
+    kernel<<<tiles, block, 0, s>>>(a, ed);
     return hipGetLastError();
 }
 

@@ -27,14 +27,13 @@ namespace gstex {
 // Texel gradients of the window route over the R x Q texels from chart row
 // ou, column ov (R, Q <= 3): window tap (row r, column q) has weight
 // A[r] * B[q], and rows and columns from R, Q on carry zero weight on every
-// valid lane.  One reduction of the R * Q * CV values of CV channels (rows of
-// `stride` channels, the first `limit` of the CV exist); the lane holding a
-// wave total adds it to its texel.
+// valid lane.  One reduction of the R * Q * CV values of CV channels (texels of
+// `stride` channels); the lane holding a wave total adds it to its texel.
 template <int R, int Q, int CV>
 __device__ __forceinline__ void window_texel_add(const float (&A)[3], const float (&B)[3],
                                                  const float (&vval)[CV], int lane,
                                                  float* vtex_chart, int ou, int ov, int h,
-                                                 int w, int stride, int limit) {
+                                                 int w, int stride) {
     float vals[R * Q * CV];
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -51,7 +50,7 @@ __device__ __forceinline__ void window_texel_add(const float (&A)[3], const floa
         const int r = rq / Q, q = rq - Q * r;
         // a window row or column past the chart edge carries no weight
         // (taps clamp inside the chart)
-        if (ou + r < h && ov + q < w && (limit >= CV || c < limit))
+        if (ou + r < h && ov + q < w)
             unsafeAtomicAdd(vtex_chart + ((ou + r) * w + (ov + q)) * stride + c, tot);
     }
 }
@@ -93,20 +92,24 @@ __device__ __forceinline__ void cotangents4(const float* src, int C, int cb, flo
 // groups of four channels: a group's reduction sums its values over the wave,
 // so a texel takes one atomic per channel however many lanes sample it.
 //   single  1x1 chart
-//   quad    every valid lane samples one texel quad: 4 taps x 4 channels
-//   window  every valid lane's taps inside one 3x3 window (2x3, 3x2 where
-//           its last row or column is out of reach)
+//   quad    every valid lane samples one texel quad,
+//   window  or its taps lie inside one 3x3 window (2x3, 3x2 where its last row
+//           or column is out of reach): matrix instructions (quad_sums), for
+//           which a lane reads channel cb + (lane & 3) of its quad's pixels
 //   lds     charts of up to kTexAccFloats values: lanes on one quad merged,
 //           then LDS adds and a flush
 //   direct  one atomic per tap and channel of the merged lanes
 // Bound by instruction issue, like the exact counts.  Before, every such chart
 // took per-lane LDS or global atomics, which serialise where the lanes of a
 // wave meet on one texel: a pass over 50k Gaussians at 800 x 600 with 8
-// channels took 4.9 ms, and 1.46 ms with these routes.
+// channels took 4.9 ms, 1.46 ms with these routes; wave reductions of the
+// quads' and windows' values took 733 us in this kernel (with blur), the matrix
+// instructions 700.
 __device__ __forceinline__ void texel_gradients_wide(
-    const float* cot, int C, float vis, const float (&wt)[4], const int (&lofs)[4], float fu,
-    float fv, int iu, int iv, int ju, int jv, bool bilinear, bool valid, uint64_t vmask, int hw,
-    int h, int w, int lane, float* acc, float* vtex_chart) {
+    const float* v_texture_out, int pid, int C, float vis, const float (&wt)[4],
+    const int (&lofs)[4], float tu, float tv, int iu, int iv, int ju, int jv, bool bilinear,
+    bool valid, uint64_t vmask, int hw, int h, int w, int lane, float* acc, float* vtex_chart) {
+    const float* const cot = v_texture_out + (size_t)pid * C;
     const int first = __ffsll((unsigned long long)vmask) - 1;
     if (hw == 1) {
         const float ws = vis * ((wt[0] + wt[1]) + (wt[2] + wt[3]));
@@ -122,50 +125,61 @@ __device__ __forceinline__ void texel_gradients_wide(
         }
         return;
     }
-    const int l0 = __builtin_amdgcn_readlane(lofs[0], first);
-    if (!(lanes_where(lofs[0] != l0) & vmask)) {
-        const int l1 = __builtin_amdgcn_readlane(lofs[1], first);
-        const int l2 = __builtin_amdgcn_readlane(lofs[2], first);
-        const int l3 = __builtin_amdgcn_readlane(lofs[3], first);
-        float wv[4];
+    // Channels cb + (lane & 3) of the four pixels of this lane's quad.
+    const int j = lane & 3;
+    const int pids[4] = {dpp_i<0x00>(pid), dpp_i<0x55>(pid), dpp_i<0xAA>(pid), dpp_i<0xFF>(pid)};
+    auto quad_values = [&](int cb, float (&value)[4]) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) wv[k] = wt[k] * vis;
-        const int code = rs_slot<16>(lane);
-        const int k = code >> 2, cc = code & 3;
-        const int at = k == 0 ? l0 : k == 1 ? l1 : k == 2 ? l2 : l3;
+        for (int m = 0; m < 4; ++m)
+            value[m] = cb + j < C ? v_texture_out[(size_t)pids[m] * C + cb + j] : 0.f;
+    };
+    // position relative to the anchor lane's taps
+    const int au = __builtin_amdgcn_readlane(iu, first);
+    const int av = __builtin_amdgcn_readlane(iv, first);
+    if (!((lanes_where(iu != au) | lanes_where(iv != av)) & vmask)) {
+        // nearest: the one tap of weight 1
+        const float y = bilinear ? tu - (float)au : ju != iu ? wt[2] + wt[3] : 0.f;
+        const float x = bilinear ? tv - (float)av : jv != iv ? wt[1] + wt[3] : 0.f;
+        QuadWeights qw;
+        qw.set(y, x, vis, lane);
+        const int t = quad_slot<4>(lane), r = (t >> 1) & 1, q = t & 1;
+        const bool own = t < 4 && au + r < h && av + q < w;
+        float* const at = vtex_chart + ((au + r) * w + av + q) * C;
         for (int cb = 0; cb < C; cb += 4) {
-            float v[4], vals[16];
-            cotangents4(cot, C, cb, v);
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) vals[4 * t + c] = wv[t] * v[c];
-            const float tot = wave_reduce_scatter(vals, lane);
-            if (code < 64 && cb + cc < C && tot != 0.f)
-                unsafeAtomicAdd(vtex_chart + at + cb + cc, tot);
+            float value[4], sums[4];
+            quad_values(cb, value);
+            quad_sums<4>(qw.w, value, sums);
+            const float tot = quad_reduce_scatter(sums, lane);
+            if (own && cb + j < C && tot != 0.f) unsafeAtomicAdd(at + cb + j, tot);
         }
         return;
     }
     if (bilinear) {
-        // window origin: the anchor lane's tap row / column, one lower when
-        // some valid lane lies below it
-        const int au = __builtin_amdgcn_readlane(iu, first);
-        const int av = __builtin_amdgcn_readlane(iv, first);
+        // window origin: one lower when some valid lane lies below the anchor
         const int ou = au - ((lanes_where(iu < au) & vmask) ? 1 : 0);
         const int ov = av - ((lanes_where(iv < av) & vmask) ? 1 : 0);
         const int ri = iu - ou, rj = ju - ou, ci = iv - ov, cj = jv - ov;
         if (!(lanes_where(((uint32_t)ri | (uint32_t)ci) > 1u) & vmask)) {
-            float A[3], B[3];
-            window_weights(1.f - fu, fu, ri, rj, A);
-            window_weights(1.f - fv, fv, ci, cj, B);
-#pragma unroll
-            for (int r = 0; r < 3; ++r) A[r] *= vis;
+            const float y = tu - (float)ou, x = tv - (float)ov;
             auto window = [&](auto R, auto Q) {
+                constexpr int NR = R.value, NQ = Q.value;
+                float a[NR];
+                row_weights(y, a);
+#pragma unroll
+                for (int r = 0; r < NR; ++r) a[r] *= vis;
+                WindowWeights<NR> ww;
+                ww.set(a, x, lane);
+                const int t = quad_slot<NR * NQ>(lane), r = (t & 63) / NQ, q = (t & 63) - NQ * r;
+                // a window row or column past the chart edge carries no weight
+                const bool own = t < NR * NQ && ou + r < h && ov + q < w;
+                float* const at = vtex_chart + ((ou + r) * w + ov + q) * C;
                 for (int cb = 0; cb < C; cb += 4) {
-                    float v[4];
-                    cotangents4(cot, C, cb, v);
-                    window_texel_add<R.value, Q.value, 4>(A, B, v, lane, vtex_chart + cb, ou, ov,
-                                                          h, w, C, C - cb);
+                    float value[4], sums[NR * NQ];
+                    quad_values(cb, value);
+#pragma unroll
+                    for (int k = 0; k < NR; ++k) quad_sums<NQ>(ww.w[k], value, sums + NQ * k);
+                    const float tot = quad_reduce_scatter(sums, lane);
+                    if (own && cb + j < C && tot != 0.f) unsafeAtomicAdd(at + cb + j, tot);
                 }
             };
             using two = std::integral_constant<int, 2>;
@@ -524,17 +538,16 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
                 if constexpr (CM <= 3) {
                     if (!(lanes_where(rj == 2) & vmask)) {
                         window_texel_add<2, 3, CM>(A, Bw, vval, lane, vtex_chart, ou, ov, s.h,
-                                                   s.w, CM, CM);
+                                                   s.w, CM);
                         return;
                     }
                     if (!(lanes_where(cj == 2) & vmask)) {
                         window_texel_add<3, 2, CM>(A, Bw, vval, lane, vtex_chart, ou, ov, s.h,
-                                                   s.w, CM, CM);
+                                                   s.w, CM);
                         return;
                     }
                 }
-                window_texel_add<3, 3, CM>(A, Bw, vval, lane, vtex_chart, ou, ov, s.h, s.w, CM,
-                                            CM);
+                window_texel_add<3, 3, CM>(A, Bw, vval, lane, vtex_chart, ou, ov, s.h, s.w, CM);
                 return;
             }
             if (tex_lds) {
@@ -561,8 +574,9 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
 #pragma unroll
                 for (int k = 0; k < 4; ++k) lofs[k] = row[k] >> kES;
                 texel_gradients_wide(
-                    cot, C, vis, wt, lofs, fu, fv, iu, iv, ju, jv, bilinear, valid, vmask, hw, s.h, s.w,
-                    lane, acc, vtex_chart);
+                    b.v_texture_out, pid, C, vis, wt, lofs, fminf((float)s.h * u, (float)(s.h - 1)),
+                    fminf((float)s.w * v, (float)(s.w - 1)), iu, iv, ju, jv, bilinear, valid,
+                    vmask, hw, s.h, s.w, lane, acc, vtex_chart);
             }
             return;
         }

@@ -387,6 +387,7 @@ constexpr int kDppQuadXor1 = 0xB1;      // quad_perm [1,0,3,2]
 constexpr int kDppQuadXor2 = 0x4E;      // quad_perm [2,3,0,1]
 constexpr int kDppRowMirror = 0x140;    // lane i <-> 15 - i within 16
 constexpr int kDppRowHalfMirror = 0x141; // lane i <-> 7 - i within 8
+constexpr int kDppRowRor4 = 0x124;      // lane i <- lane (i + 4) mod 16 within 16
 constexpr int kDppRowRor8 = 0x128;      // lane i <- lane (i + 8) mod 16 within 16 (= i ^ 8)
 
 template <int CTRL>
@@ -539,6 +540,135 @@ __device__ __forceinline__ int rs_slot(int lane) {
         if (pos < h) pos += bit ? np : 0;
         else dup |= bit;
     }
+    return pos | (dup << 6);
+}
+
+// ------------------------------------------------------------------ texel sums on matrix cores
+// The texel sums of a wave over an R x Q texel window,
+//   sum over pixels of A[r] B[q] value[c],
+// are a product of a (texels x 64) and a (64 x channels) matrix.  The 4x4x1
+// matrix instruction of 16 blocks takes it as it lies in the registers: block b
+// is the lane quad 4b .. 4b + 3, whose pixels m = 0..3 are four steps, row i of
+// a step is the weight of window column i (held by the quad's lane i), column j
+// the value of channel j (held by lane j).  So a window row takes four matrix
+// instructions for any Q <= 4 and four channels, after which lane j of quad b
+// holds channel j of the quad's sums and only the 16 quads are left to add.
+
+// Value of lane m of this lane's quad.
+template <int M>
+__device__ __forceinline__ float quad_lane(float v) {
+    return dpp<M * 0x55>(v);
+}
+
+// Bilinear weight of texel row (column) c at position p along it, both
+// relative to the window: the smaller of p - (c - 1) and (c + 1) - p, at least
+// zero (both sides come out as 1 - fract and fract do, without rounding p).
+__device__ __forceinline__ float tap_weight(float p, float c_below, float c_above) {
+    return __builtin_amdgcn_fmed3f(0.f, p - c_below, c_above - p);
+}
+
+// Weights of the window's columns in the layout above: lane i of a quad holds,
+// for each of the quad's four pixels m, a[r] B[i] of that pixel, with a[r] its
+// row weights (row_weights) and x its column position relative to the window (a
+// pixel that adds nothing: x far outside, where every column's weight is zero).
+template <int R>
+__device__ __forceinline__ void row_weights(float y, float (&a)[R]) {
+    if constexpr (R == 2) {  // y in [0, 1]
+        a[0] = 1.f - y;
+        a[1] = y;
+    } else {
+#pragma unroll
+        for (int r = 0; r < R; ++r) a[r] = tap_weight(y, (float)(r - 1), (float)(r + 1));
+    }
+}
+
+template <int R>
+struct WindowWeights {
+    float w[R][4];
+    __device__ __forceinline__ void set(const float (&a)[R], float x, int lane) {
+        const float col = (float)(lane & 3);
+        step<0>(a, x, col);
+        step<1>(a, x, col);
+        step<2>(a, x, col);
+        step<3>(a, x, col);
+    }
+    template <int M>
+    __device__ __forceinline__ void step(const float (&a)[R], float x, float col) {
+        const float t = tap_weight(quad_lane<M>(x), col - 1.f, col + 1.f);
+#pragma unroll
+        for (int r = 0; r < R; ++r) w[r][M] = quad_lane<M>(a[r]) * t;
+    }
+};
+
+// The same for one texel quad, y and x in [0, 1]: lane i of a pixel quad holds
+// the weights of texel (i >> 1, i & 1), times each pixel's scale.
+struct QuadWeights {
+    float w[4];
+    __device__ __forceinline__ void set(float y, float x, float scale, int lane) {
+        const float row = lane & 2 ? 0.f : 1.f, col = lane & 1 ? 0.f : 1.f;
+        step<0>(y, x, scale, row, col);
+        step<1>(y, x, scale, row, col);
+        step<2>(y, x, scale, row, col);
+        step<3>(y, x, scale, row, col);
+    }
+    template <int M>
+    __device__ __forceinline__ void step(float y, float x, float scale, float row, float col) {
+        // |t - 1| is 1 - t, |t - 0| is t
+        w[M] = quad_lane<M>(scale) *
+               (fabsf(quad_lane<M>(y) - row) * fabsf(quad_lane<M>(x) - col));
+    }
+};
+
+using MfmaAcc = __attribute__((__vector_size__(4 * sizeof(float)))) float;
+
+// Sums over the quad's pixels of weight x channel: sums[i] on lane j is that of
+// lane i's weights (one window row) and channel j; value[m] is channel j of
+// pixel m.
+template <int Q>
+__device__ __forceinline__ void quad_sums(const float (&w)[4], const float (&value)[4],
+                                          float* sums) {
+    MfmaAcc acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+        acc = __builtin_amdgcn_mfma_f32_4x4x1f32(w[m], value[m], acc, 0, 0, 0);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) sums[q] = acc[q];
+}
+
+// Sums of N <= 16 values over the 16 quads of a wave (the four lanes of a quad
+// hold unrelated sums): two halving rounds over lane bits 5 and 4, then plain
+// sums over bits 3 and 2, by which a lane picks one of the up to four values
+// left.  Which value a lane ends with, quad_slot<N> (bit 6: another quad
+// with lower bits holds it too).
+template <int N>
+__device__ __forceinline__ float quad_reduce_scatter(const float (&v)[N], int lane) {
+    constexpr int N1 = N - N / 2, N2 = N1 - N1 / 2;
+    static_assert(N2 <= 4, "at most 16 values");
+    float w[N1], x[N2];
+#pragma unroll
+    for (int k = 0; k < N1; ++k) w[k] = swap32_sum(v[k], v[k + N1 < N ? k + N1 : k]);
+#pragma unroll
+    for (int k = 0; k < N2; ++k) {
+        x[k] = swap16_sum(w[k], w[k + N2 < N1 ? k + N2 : k]);
+        x[k] += dpp<kDppRowRor8>(x[k]);
+        x[k] += dpp<kDppRowRor4>(x[k]);
+    }
+    float r = x[0];
+#pragma unroll
+    for (int k = 1; k < N2; ++k) r = ((lane >> 2) & 3) == k ? x[k] : r;
+    return r;
+}
+
+template <int N>
+__device__ __forceinline__ int quad_slot(int lane) {
+    constexpr int N1 = N - N / 2, N2 = N1 - N1 / 2;
+    int pos = (lane >> 2) & 3;
+    int dup = pos >= N2 ? 1 : 0;
+    const int b4 = (lane >> 4) & 1, b5 = (lane >> 5) & 1;
+    if (pos < N1 / 2) pos += b4 ? N2 : 0;
+    else dup |= b4;
+    if (pos < N / 2) pos += b5 ? N1 : 0;
+    else dup |= b5;
     return pos | (dup << 6);
 }
 
