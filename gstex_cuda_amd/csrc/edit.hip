@@ -111,18 +111,8 @@ __attribute__((amdgpu_waves_per_eu(PRECISE ? 1 : 5))) void k_texture_edit(Raster
     // channels 0..3 of the pixels of this lane's quad, channel lane & 3
     float quad_val[4];
     {
-        const int c = lane & 3;
-        auto pick = [&](float v0, float v1, float v2, float v3) {
-            return c == 0 ? v0 : c == 1 ? v1 : c == 2 ? v2 : v3;
-        };
-#define GSTEX_QUAD_VAL(M)                                                                       \
-    quad_val[M] = pick(quad_lane<M>(val[0]), quad_lane<M>(val[1]), quad_lane<M>(val[2]),        \
-                       quad_lane<M>(val[3]))
-        GSTEX_QUAD_VAL(0);
-        GSTEX_QUAD_VAL(1);
-        GSTEX_QUAD_VAL(2);
-        GSTEX_QUAD_VAL(3);
-#undef GSTEX_QUAD_VAL
+        const float rgba[4] = {val[0], val[1], val[2], val[3]};
+        quad_transpose(rgba, lane, quad_val);
     }
 
     // One list entry: Gaussian g with record s.  The pair math runs for every

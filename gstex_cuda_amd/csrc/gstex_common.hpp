@@ -50,16 +50,16 @@ enum GradSlot : int {
     G_P12 = 5,    //        sum vl1 * l2
     G_P21 = 6,    //        sum vl2 * l1
     G_P22 = 7,    //        sum vl2 * l2
-    G_U1 = 8,     //        sum vu * l1
-    G_U2 = 9,     //        sum vu * l2
-    G_V1 = 10,    //        sum vv * l1
-    G_V2 = 11,    //        sum vv * l2
-    G_VL1 = 12,   //        sum vl1
-    G_VL2 = 13,   //        sum vl2
-    G_VU = 14,    //        sum vu
-    G_VV = 15,    //        sum vv
-    G_VNUM = 16,  //        sum vnum
-    G_AX3X = 17,  // 17..19 sum vden * ray + vis * dL/dnormal
+    G_VL1 = 8,    //        sum vl1
+    G_VL2 = 9,    //        sum vl2
+    G_VNUM = 10,  //        sum vnum
+    G_AX3X = 11,  // 11..13 sum vden * ray + vis * dL/dnormal
+    G_U1 = 14,    //        sum vu * l1 (this and the next five: charts of
+    G_U2 = 15,    //        sum vu * l2  more than one texel only)
+    G_V1 = 16,    //        sum vv * l1
+    G_V2 = 17,    //        sum vv * l2
+    G_VU = 18,    //        sum vu
+    G_VV = 19,    //        sum vv
     G_EXTRA = 20, // 20..31 texel gradients carried through the same reduction
     G_PIX = 30,   // 30..31 d/d projected mean (blur term)
     kGradFloats = 32

@@ -87,81 +87,135 @@ __device__ __forceinline__ void cotangents4(const float* src, int C, int cb, flo
     }
 }
 
-// Texel gradients of a chart with a runtime count C of more than four
-// channels; cot is this pixel's row of texture cotangents.  The routes are those of the exact channel counts, over
-// groups of four channels: a group's reduction sums its values over the wave,
-// so a texel takes one atomic per channel however many lanes sample it.
-//   single  1x1 chart
+// Texel gradients of a chart of more than one texel with C channels (exact
+// count CM <= 4, else the runtime count in groups of four), cotangents vtex of
+// this pixel, quad_val of its lane quad (CM <= 4), by a wave-uniform choice.  A
+// group's sums run over the wave, so a texel takes one atomic per channel
+// however many lanes sample it.
 //   quad    every valid lane samples one texel quad,
-//   window  or its taps lie inside one 3x3 window (2x3, 3x2 where its last row
-//           or column is out of reach): matrix instructions (quad_sums), for
-//           which a lane reads channel cb + (lane & 3) of its quad's pixels
+//   window  or (bilinear) its taps lie inside one 3x3 window (2x3, 3x2 where its
+//           last row or column is out of reach): matrix instructions for four and
+//           more channels (quad_sums; a lane reads channel cb + (lane & 3) of
+//           its quad's pixels), wave reductions for up to three
 //   lds     charts of up to kTexAccFloats values: lanes on one quad merged,
 //           then LDS adds and a flush
-//   direct  one atomic per tap and channel of the merged lanes
-// Bound by instruction issue, like the exact counts.  Before, every such chart
-// took per-lane LDS or global atomics, which serialise where the lanes of a
-// wave meet on one texel: a pass over 50k Gaussians at 800 x 600 with 8
-// channels took 4.9 ms, 1.46 ms with these routes; wave reductions of the
-// quads' and windows' values took 733 us in this kernel (with blur), the matrix
-// instructions 700.
-__device__ __forceinline__ void texel_gradients_wide(
-    const float* v_texture_out, int pid, int C, float vis, const float (&wt)[4],
-    const int (&lofs)[4], float tu, float tv, int iu, int iv, int ju, int jv, bool bilinear,
-    bool valid, uint64_t vmask, int hw, int h, int w, int lane, float* acc, float* vtex_chart) {
+//   direct  one atomic per tap and channel
+// Bound by instruction issue.  A pass over 50k Gaussians at 800 x 600 with 8
+// channels took 4.9 ms with per-lane LDS or global atomics, which serialise
+// where the lanes of a wave meet on one texel, 1.46 ms with these routes; wave
+// reductions of the quads' and windows' values took 733 us in this kernel (with
+// blur), the matrix instructions 700.  Four channels, 50k Gaussians at 1600 x 1200: 774 us by
+// wave reductions, 658; three or fewer gain nothing (985 us either way at 1080p,
+// 500k Gaussians).
+template <int CM>
+__device__ __forceinline__ void texel_gradients(
+    const float (&vtex)[CM <= 4 ? CM : 1], const float (&quad_val)[4], const float* v_texture_out,
+    int pid, int C, float vis, const float (&wt)[4], const int (&lofs)[4], float fu, float fv,
+    float tu, float tv, int iu, int iv, int ju, int jv, bool bilinear, bool valid, uint64_t vmask,
+    int h, int w, int lane, float* acc, float* vtex_chart) {
+    constexpr int G = CM <= 4 ? CM : 4;
     const float* const cot = v_texture_out + (size_t)pid * C;
     const int first = __ffsll((unsigned long long)vmask) - 1;
-    if (hw == 1) {
-        const float ws = vis * ((wt[0] + wt[1]) + (wt[2] + wt[3]));
-        const int code = rs_slot<4>(lane);
-        for (int cb = 0; cb < C; cb += 4) {
-            float v[4];
+    auto values = [&](int cb, float (&v)[G]) {
+        if constexpr (CM <= 4) {
+#pragma unroll
+            for (int c = 0; c < G; ++c) v[c] = vtex[c];
+        } else {
             cotangents4(cot, C, cb, v);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) v[c] *= ws;
-            const float tot = wave_reduce_scatter(v, lane);
-            if (code < 64 && cb + code < C && tot != 0.f)
-                unsafeAtomicAdd(vtex_chart + cb + code, tot);
         }
-        return;
-    }
-    // Channels cb + (lane & 3) of the four pixels of this lane's quad.
-    const int j = lane & 3;
-    const int pids[4] = {dpp_i<0x00>(pid), dpp_i<0x55>(pid), dpp_i<0xAA>(pid), dpp_i<0xFF>(pid)};
-    auto quad_values = [&](int cb, float (&value)[4]) {
-#pragma unroll
-        for (int m = 0; m < 4; ++m)
-            value[m] = cb + j < C ? v_texture_out[(size_t)pids[m] * C + cb + j] : 0.f;
     };
-    // position relative to the anchor lane's taps
+    // position relative to the anchor lane's taps; window origin one lower
+    // when some valid lane lies below it
     const int au = __builtin_amdgcn_readlane(iu, first);
     const int av = __builtin_amdgcn_readlane(iv, first);
-    if (!((lanes_where(iu != au) | lanes_where(iv != av)) & vmask)) {
-        // nearest: the one tap of weight 1
-        const float y = bilinear ? tu - (float)au : ju != iu ? wt[2] + wt[3] : 0.f;
-        const float x = bilinear ? tv - (float)av : jv != iv ? wt[1] + wt[3] : 0.f;
-        QuadWeights qw;
-        qw.set(y, x, vis, lane);
-        const int t = quad_slot<4>(lane), r = (t >> 1) & 1, q = t & 1;
-        const bool own = t < 4 && au + r < h && av + q < w;
-        float* const at = vtex_chart + ((au + r) * w + av + q) * C;
-        for (int cb = 0; cb < C; cb += 4) {
-            float value[4], sums[4];
-            quad_values(cb, value);
-            quad_sums<4>(qw.w, value, sums);
-            const float tot = quad_reduce_scatter(sums, lane);
-            if (own && cb + j < C && tot != 0.f) unsafeAtomicAdd(at + cb + j, tot);
-        }
-        return;
+    const bool quad = !((lanes_where(iu != au) | lanes_where(iv != av)) & vmask);
+    int ou = au, ov = av;
+    bool window = false;
+    if (!quad && bilinear) {
+        ou = au - ((lanes_where(iu < au) & vmask) ? 1 : 0);
+        ov = av - ((lanes_where(iv < av) & vmask) ? 1 : 0);
+        window = !(lanes_where(((uint32_t)(iu - ou) | (uint32_t)(iv - ov)) > 1u) & vmask);
     }
-    if (bilinear) {
-        // window origin: one lower when some valid lane lies below the anchor
-        const int ou = au - ((lanes_where(iu < au) & vmask) ? 1 : 0);
-        const int ov = av - ((lanes_where(iv < av) & vmask) ? 1 : 0);
-        const int ri = iu - ou, rj = ju - ou, ci = iv - ov, cj = jv - ov;
-        if (!(lanes_where(((uint32_t)ri | (uint32_t)ci) > 1u) & vmask)) {
+    const int rj = ju - ou, cj = jv - ov;
+    if constexpr (CM <= 3) {
+        float vval[CM];
+#pragma unroll
+        for (int c = 0; c < CM; ++c) vval[c] = vis * vtex[c];
+        if (quad) {
+            float vals[4 * CM];
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int c = 0; c < CM; ++c) vals[CM * k + c] = wt[k] * vval[c];
+            const float tot = wave_reduce_scatter(vals, lane);
+            const int code = rs_slot<4 * CM>(lane);
+            // the anchor lane's tap rows (every valid lane's quad), read here
+            // while every lane is active
+            const int row0 = __builtin_amdgcn_readlane(lofs[0], first);
+            const int row1 = __builtin_amdgcn_readlane(lofs[1], first);
+            const int row2 = __builtin_amdgcn_readlane(lofs[2], first);
+            const int row3 = __builtin_amdgcn_readlane(lofs[3], first);
+            if (code < 64 && tot != 0.f) {
+                const int k = code / CM, c = code - CM * k;
+                const int rr = k == 0 ? row0 : k == 1 ? row1 : k == 2 ? row2 : row3;
+                unsafeAtomicAdd(vtex_chart + rr + c, tot);
+            }
+            return;
+        }
+        if (window) {
+            // separable weights: tap (row r, column q) has weight A[r] * B[q];
+            // rows iu, ju and columns iv, jv relative to the origin lie in 0..2
+            // (ju = iu at the chart edge).  When no valid lane's taps reach
+            // row (column) 2, the window is 2 x 3 (3 x 2).
+            float A[3], B[3];
+            window_weights(1.f - fu, fu, iu - ou, rj, A);
+            window_weights(1.f - fv, fv, iv - ov, cj, B);
+            if (!(lanes_where(rj == 2) & vmask))
+                window_texel_add<2, 3, CM>(A, B, vval, lane, vtex_chart, ou, ov, h, w, CM);
+            else if (!(lanes_where(cj == 2) & vmask))
+                window_texel_add<3, 2, CM>(A, B, vval, lane, vtex_chart, ou, ov, h, w, CM);
+            else
+                window_texel_add<3, 3, CM>(A, B, vval, lane, vtex_chart, ou, ov, h, w, CM);
+            return;
+        }
+    } else {
+        // channels cb + (lane & 3) of the four pixels of this lane's quad
+        const int j = lane & 3;
+        int pids[4] = {0, 0, 0, 0};
+        if constexpr (CM > 4) {
+            pids[0] = dpp_i<0x00>(pid);
+            pids[1] = dpp_i<0x55>(pid);
+            pids[2] = dpp_i<0xAA>(pid);
+            pids[3] = dpp_i<0xFF>(pid);
+        }
+        auto quad_values = [&](int cb, float (&value)[4]) {
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                if constexpr (CM <= 4) value[m] = quad_val[m];
+                else value[m] = cb + j < C ? v_texture_out[(size_t)pids[m] * C + cb + j] : 0.f;
+            }
+        };
+        if (quad) {
+            // nearest: the one tap of weight 1
+            const float y = bilinear ? tu - (float)au : ju != iu ? wt[2] + wt[3] : 0.f;
+            const float x = bilinear ? tv - (float)av : jv != iv ? wt[1] + wt[3] : 0.f;
+            QuadWeights qw;
+            qw.set(y, x, vis, lane);
+            const int t = quad_slot<4>(lane), r = (t >> 1) & 1, q = t & 1;
+            const bool own = t < 4 && au + r < h && av + q < w;
+            float* const at = vtex_chart + ((au + r) * w + av + q) * C;
+            for (int cb = 0; cb < C; cb += 4) {
+                float value[4], sums[4];
+                quad_values(cb, value);
+                quad_sums<4>(qw.w, value, sums);
+                const float tot = quad_reduce_scatter(sums, lane);
+                if (own && cb + j < C && tot != 0.f) unsafeAtomicAdd(at + cb + j, tot);
+            }
+            return;
+        }
+        if (window) {
             const float y = tu - (float)ou, x = tv - (float)ov;
-            auto window = [&](auto R, auto Q) {
+            auto add = [&](auto R, auto Q) {
                 constexpr int NR = R.value, NQ = Q.value;
                 float a[NR];
                 row_weights(y, a);
@@ -184,19 +238,29 @@ __device__ __forceinline__ void texel_gradients_wide(
             };
             using two = std::integral_constant<int, 2>;
             using three = std::integral_constant<int, 3>;
-            if (!(lanes_where(rj == 2) & vmask)) window(two{}, three{});
-            else if (!(lanes_where(cj == 2) & vmask)) window(three{}, two{});
-            else window(three{}, three{});
+            if (!(lanes_where(rj == 2) & vmask)) add(two{}, three{});
+            else if (!(lanes_where(cj == 2) & vmask)) add(three{}, two{});
+            else add(three{}, three{});
             return;
         }
     }
-    const QuadMerge qm = quad_merge_setup(valid ? lofs[0] : -1, lane);
-    const bool lds = hw * C <= kTexAccFloats;
-    for (int cb = 0; cb < C; cb += 4) {
-        float v[4];
-        cotangents4(cot, C, cb, v);
+    const bool lds = h * w * C <= kTexAccFloats;
+    if (CM <= 4 && !lds) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < G; ++c)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float add = wt[k] * (vis * vtex[CM <= 4 ? c : 0]);
+                if (add != 0.f) unsafeAtomicAdd(vtex_chart + lofs[k] + c, add);
+            }
+        return;
+    }
+    const QuadMerge qm = quad_merge_setup(valid ? lofs[0] : -1, lane);
+    for (int cb = 0; cb < C; cb += 4) {
+        float v[G];
+        values(cb, v);
+#pragma unroll
+        for (int c = 0; c < G; ++c) {
             float q[4];
 #pragma unroll
             for (int k = 0; k < 4; ++k) q[k] = quad_merge(wt[k] * (vis * v[c]), qm);
@@ -290,6 +354,8 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
         vT = a.background[0] * vo.x + a.background[1] * vo.y + a.background[2] * vo.z -
              b.v_alpha[pid];
     }
+    float quad_val[4] = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (CM == 4) quad_transpose(vtex, lane, quad_val);
     int r0, r1;
     tile_range(a, tile, r0, r1);
     // Entries past the wave's last contributing index are dead for every lane.
@@ -301,66 +367,25 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
     const float tn = 0.01f, tf = 1000.0f;
     const int last_e = inside ? bfin : -1;  // entries up to it may contribute
 
-    // One list entry (wave-uniform index e, Gaussian g with record s).
-    auto entry = [&](const int e, const int g, const Splat& s) {
-        // The pair math and the taps run for every lane: they are finite for
-        // any pixel ray, and tap offsets stay inside the chart.  A lane that
-        // does not contribute keeps T and vT and gets zero seeds (vis, valpha,
-        // vt, vu, vv), so every gradient value below is zero for it without a
-        // branch or per-value selects.
-        const Pair p = pair_eval(s, pr, use_blur, PRECISE && a.precise_edge);
-        const bool valid = e <= last_e && !p.skip;
-        const uint64_t vmask = lanes_where(e <= last_e) & ~skip_lanes(p);
-        if (vmask == 0) return;
-
-        // Transmittance before this Gaussian (1 - alpha >= 0.01) and the texel taps.
-        const Chart ch = chart_of<TB>(a.texture, s, C, a.num_texels);
-        // (a reciprocal and a product: about 1.5 ulp per entry, 3e-6 relative
-        // after a thousand)
-        if (valid) T = T * __builtin_amdgcn_rcpf(1.f - p.alpha);
-        const float vis = valid ? p.alpha * T : 0.f;
-        float u, v, wt[4], fu, fv;
+    // The gradients of one entry, given its pair and visibility.
+    auto pixels = [&](const int e, const int g, const Splat& s, const Pair& p, const Chart& ch,
+                      const bool valid, const uint64_t vmask, const float vis, auto flat_c) {
+        constexpr bool FLAT = decltype(flat_c)::value;
+        float wt[4], fu, fv, u = 0.f, v = 0.f;
         int row[4];  // byte offsets inside the chart
         int iu, iv, ju, jv;  // tap rows (u) and columns (v) of the chart
         splat_uv(s, p.delta, u, v);
-        chart_taps_ij(s, ch, u, v, bilinear, wt, row, fu, fv, iu, iv, ju, jv);
-        // How the texel gradients reach HBM (wave-uniform choice; with more
-        // than four channels in texel_gradients_wide):
-        //   single  1x1 chart: C values in the reduction
-        //   quad    every valid lane samples the same texel quad, C <= 3:
-        //           4 taps x C values in the reduction
-        //   window  bilinear, C <= 4, every valid lane's taps inside one 3x3
-        //           texel window: the 9 C separable weight products in the
-        //           reduction
-        //   lds     chart of <= kTexAccFloats values: LDS accumulation + flush
-        //   direct  one atomic per tap
-        const int first = __ffsll((unsigned long long)vmask) - 1;
-        const int hw = ch.ok ? s.h * s.w : 0;
-        const bool tex_single = CM <= 4 && hw == 1;
-        const int row0 = __builtin_amdgcn_readlane(row[0], first);
-        const bool quad32 = CM <= 3 && ch.ok && !tex_single &&
-                            !(lanes_where(row[0] != row0) & vmask);
-        // window origin (ou, ov): the anchor lane's tap row / column, one
-        // lower when some valid lane lies below it (formed only where the
-        // window route is open)
-        int ou = 0, ov = 0;
-        bool win3 = false;
-        if (CM <= 4 && ch.ok && !tex_single && !quad32 && bilinear && C >= 1) {
-            const int au = __builtin_amdgcn_readlane(iu, first);
-            const int av = __builtin_amdgcn_readlane(iv, first);
-            ou = au - ((lanes_where(iu < au) & vmask) ? 1 : 0);
-            ov = av - ((lanes_where(iv < av) & vmask) ? 1 : 0);
-            win3 = !(lanes_where(((uint32_t)(iu - ou) | (uint32_t)(iv - ov)) > 1u) & vmask);
+        if constexpr (FLAT) {
+            tap_weights(s, u, v, bilinear, wt);  // they sum to one up to rounding
+        } else {
+            chart_taps_ij(s, ch, u, v, bilinear, wt, row, fu, fv, iu, iv, ju, jv);
         }
-        const bool tex_lds = CM <= 4 && ch.ok && !tex_single && !quad32 && !win3 && C > 0 &&
-                             hw * C <= kTexAccFloats;
         float* const vtex_chart = b.v_texture + (size_t)(ch.ok ? s.start : 0) * C;
 
-        // The per-Gaussian values (GradSlot 0..19, then the two blur values
-        // in the general kernels) and the texel terms of the routes.
-        constexpr int NB = G_EXTRA + (GENERAL ? 2 : 0);
+        // The per-Gaussian values: GradSlot 0..19 (to G_U1 for one texel),
+        // then the two blur values in the general kernels.
+        constexpr int NG = FLAT ? (int)G_U1 : (int)G_EXTRA, NB = NG + (GENERAL ? 2 : 0);
         float gr[NB];
-        float vval[CM <= 4 ? CM : 1];  // vis * dL/dtexture_out per channel
         {
             gr[G_RGB + 0] = vis * vo.x;
             gr[G_RGB + 1] = vis * vo.y;
@@ -373,58 +398,60 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
             // (texture_helpers.cuh:262-299) takes tap differences, which are
             // differences of two D: coincident taps (equal texels) give equal
             // D and exactly zero.
-            float D[4] = {0.f, 0.f, 0.f, 0.f};
-            if constexpr (CM <= 4) {
-                float tv[4][CM];  // all taps loaded before use
+            if constexpr (FLAT) {
+                float d0 = 0.f;
+                if constexpr (CM <= 4) {
 #pragma unroll
-                for (int k = 0; k < 4; ++k)
+                    for (int c = 0; c < CM; ++c) d0 = fmaf(chart_texel<TB>(ch, c * E), vtex[c], d0);
+                } else {
+                    for (int c = 0; c < C; ++c) d0 = fmaf(chart_texel<TB>(ch, c * E), cot[c], d0);
+                }
+                vvis += (wt[0] * d0 + wt[1] * d0) + (wt[2] * d0 + wt[3] * d0);
+            } else {
+                float D[4] = {0.f, 0.f, 0.f, 0.f};
+                if constexpr (CM <= 4) {
+                    float tv[4][CM];  // all taps loaded before use
 #pragma unroll
-                    for (int c = 0; c < CM; ++c) tv[k][c] = chart_texel<TB>(ch, row[k] + c * E);
+                    for (int k = 0; k < 4; ++k)
 #pragma unroll
-                for (int c = 0; c < CM; ++c) {
+                        for (int c = 0; c < CM; ++c) tv[k][c] = chart_texel<TB>(ch, row[k] + c * E);
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) D[k] = fmaf(tv[k][c], vtex[c], D[k]);
-                    vval[c] = vis * vtex[c];
-                    if (!tex_single && !quad32 && !win3 && !tex_lds && ch.ok) {
+                    for (int c = 0; c < CM; ++c)
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) D[k] = fmaf(tv[k][c], vtex[c], D[k]);
+                } else {
+                    // groups of four channels, a full group's taps in wide loads
+                    for (int cb = 0; cb < C; cb += 4) {
+                        float v4[4], tv[4][4];
+                        cotangents4(cot, C, cb, v4);
 #pragma unroll
                         for (int k = 0; k < 4; ++k) {
-                            const float add = wt[k] * vval[c];
-                            if (add != 0.f) unsafeAtomicAdd(vtex_chart + (row[k] >> kES) + c, add);
+                            if (cb + 4 <= C) {
+#pragma unroll
+                                for (int c = 0; c < 4; ++c)
+                                    tv[k][c] = chart_texel<TB>(ch, row[k] + (cb + c) * E);
+                            } else {
+#pragma unroll
+                                for (int c = 0; c < 4; ++c)
+                                    tv[k][c] = cb + c < C
+                                                   ? chart_texel<TB>(ch, row[k] + (cb + c) * E)
+                                                   : 0.f;
+                            }
                         }
+#pragma unroll
+                        for (int c = 0; c < 4; ++c)
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) D[k] = fmaf(tv[k][c], v4[c], D[k]);
                     }
                 }
-            } else {
-                // groups of four channels, a full group's taps in wide loads
-                for (int cb = 0; cb < C; cb += 4) {
-                    float v[4], tv[4][4];
-                    cotangents4(cot, C, cb, v);
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        if (cb + 4 <= C) {
-#pragma unroll
-                            for (int c = 0; c < 4; ++c)
-                                tv[k][c] = chart_texel<TB>(ch, row[k] + (cb + c) * E);
-                        } else {
-#pragma unroll
-                            for (int c = 0; c < 4; ++c)
-                                tv[k][c] = cb + c < C
-                                               ? chart_texel<TB>(ch, row[k] + (cb + c) * E)
-                                               : 0.f;
-                        }
-                    }
-#pragma unroll
-                    for (int c = 0; c < 4; ++c)
-#pragma unroll
-                        for (int k = 0; k < 4; ++k) D[k] = fmaf(tv[k][c], v[c], D[k]);
+                vvis += (wt[0] * D[0] + wt[1] * D[1]) + (wt[2] * D[2] + wt[3] * D[3]);
+                if (bilinear && prop_uv) {
+                    vu = vis * (float)s.h * ((1.f - fv) * (D[2] - D[0]) + fv * (D[3] - D[1]));
+                    vv = vis * (float)s.w * ((1.f - fu) * (D[1] - D[0]) + fu * (D[3] - D[2]));
                 }
-            }
-            vvis += (wt[0] * D[0] + wt[1] * D[1]) + (wt[2] * D[2] + wt[3] * D[3]);
-            if (bilinear && prop_uv) {
-                vu = vis * (float)s.h * ((1.f - fv) * (D[2] - D[0]) + fv * (D[3] - D[1]));
-                vv = vis * (float)s.w * ((1.f - fu) * (D[1] - D[0]) + fu * (D[3] - D[2]));
             }
 
-            if (!valid) vu = vv = 0.f;  // NaN-safe zero seeds
+            if (!FLAT && !valid) vu = vv = 0.f;  // NaN-safe zero seeds
             const float dvis = vvis - vT;
             float valpha = T * dvis;
             float vTcur = fmaf(p.alpha, dvis, vT);  // alpha vvis + (1 - alpha) vT
@@ -447,9 +474,12 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
             const float vsigma = p.blur_sel ? 0.f : -s.opac * p.G * valpha;
             const float vl1 = vsigma * s.iq1 * p.l1;
             const float vl2 = vsigma * s.iq2 * p.l2;
-            const V3 vdelta = v3(vl1 * s.a1.x + vl2 * s.a2.x + s.umap.x * vu + s.vmap.x * vv,
-                                 vl1 * s.a1.y + vl2 * s.a2.y + s.umap.y * vu + s.vmap.y * vv,
-                                 vl1 * s.a1.z + vl2 * s.a2.z + s.umap.z * vu + s.vmap.z * vv);
+            V3 vdelta = v3(vl1 * s.a1.x + vl2 * s.a2.x, vl1 * s.a1.y + vl2 * s.a2.y,
+                           vl1 * s.a1.z + vl2 * s.a2.z);
+            if constexpr (!FLAT)
+                vdelta = v3(vdelta.x + s.umap.x * vu + s.vmap.x * vv,
+                            vdelta.y + s.umap.y * vu + s.vmap.y * vv,
+                            vdelta.z + s.umap.z * vu + s.vmap.z * vv);
             vt += dot3(vdelta, pr.r);
             const float vnum = vt * __builtin_amdgcn_rcpf(p.den);
             const float vden = -vnum * p.t;
@@ -457,18 +487,20 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
             gr[G_P12] = vl1 * p.l2;
             gr[G_P21] = vl2 * p.l1;
             gr[G_P22] = vl2 * p.l2;
-            gr[G_U1] = vu * p.l1;
-            gr[G_U2] = vu * p.l2;
-            gr[G_V1] = vv * p.l1;
-            gr[G_V2] = vv * p.l2;
             gr[G_VL1] = vl1;
             gr[G_VL2] = vl2;
-            gr[G_VU] = vu;
-            gr[G_VV] = vv;
             gr[G_VNUM] = vnum;
             gr[G_AX3X + 0] = vden * pr.r.x + vis * vn.x;
             gr[G_AX3X + 1] = vden * pr.r.y + vis * vn.y;
             gr[G_AX3X + 2] = vden * pr.r.z + vis * vn.z;
+            if constexpr (!FLAT) {
+                gr[G_U1] = vu * p.l1;
+                gr[G_U2] = vu * p.l2;
+                gr[G_V1] = vv * p.l1;
+                gr[G_V2] = vv * p.l2;
+                gr[G_VU] = vu;
+                gr[G_VV] = vv;
+            }
             if constexpr (GENERAL) {
                 float px = 0.f, py = 0.f;
                 if (use_blur) {
@@ -476,8 +508,8 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
                     px = 2.0f * vsb * (s.pix_x - pr.px);
                     py = 2.0f * vsb * (s.pix_y - pr.py);
                 }
-                gr[G_EXTRA] = px;
-                gr[G_EXTRA + 1] = py;
+                gr[NG] = px;
+                gr[NG + 1] = py;
             }
         }
 
@@ -490,117 +522,62 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
             const float tot = wave_reduce_scatter(gr, lane);
             const int code = rs_slot<NB>(lane);
             if (code < 64 && tot != 0.f)
-                unsafeAtomicAdd(grec + (code < G_EXTRA ? code : G_PIX + (code - G_EXTRA)), tot);
+                unsafeAtomicAdd(grec + (code < NG ? code : G_PIX + (code - NG)), tot);
         }
-        if constexpr (CM <= 4) {
-            if (tex_single) {
-                float vals[CM];
-                const float wsum = (wt[0] + wt[1]) + (wt[2] + wt[3]);
+        if (!ch.ok) return;
+        if constexpr (FLAT) {
+            constexpr int G = CM <= 4 ? CM : 4;
+            const int code = rs_slot<G>(lane);
+            const float wsum = (wt[0] + wt[1]) + (wt[2] + wt[3]);
+            for (int cb = 0; cb < C; cb += 4) {
+                float vals[G];
+                if constexpr (CM <= 4) {
 #pragma unroll
-                for (int c = 0; c < CM; ++c) vals[c] = wsum * vval[c];
+                    for (int c = 0; c < G; ++c) vals[c] = wsum * (vis * vtex[c]);
+                } else {
+                    cotangents4(cot, C, cb, vals);
+#pragma unroll
+                    for (int c = 0; c < G; ++c) vals[c] *= vis * wsum;
+                }
                 const float tot = wave_reduce_scatter(vals, lane);
-                const int code = rs_slot<CM>(lane);
-                if (code < 64 && tot != 0.f) unsafeAtomicAdd(vtex_chart + code, tot);
-                return;
+                if (code < 64 && cb + code < C && tot != 0.f)
+                    unsafeAtomicAdd(vtex_chart + cb + code, tot);
             }
-            if (quad32) {
-                constexpr int QC = CM <= 3 ? CM : 3;
-                float vals[4 * QC];
+        } else {
+            int lofs[4];
 #pragma unroll
-                for (int k = 0; k < 4; ++k)
-#pragma unroll
-                    for (int c = 0; c < QC; ++c) vals[QC * k + c] = wt[k] * vval[c];
-                const float tot = wave_reduce_scatter(vals, lane);
-                const int code = rs_slot<4 * QC>(lane);
-                // the anchor lane's other tap rows (every valid lane's quad),
-                // read here while every lane is active
-                const int row1 = __builtin_amdgcn_readlane(row[1], first);
-                const int row2 = __builtin_amdgcn_readlane(row[2], first);
-                const int row3 = __builtin_amdgcn_readlane(row[3], first);
-                if (code < 64 && tot != 0.f) {
-                    const int k = code / QC, c = code - QC * k;
-                    const int rr = k == 0 ? row0 : k == 1 ? row1 : k == 2 ? row2 : row3;
-                    unsafeAtomicAdd(vtex_chart + (rr >> kES) + c, tot);
-                }
-                return;
-            }
-            if (win3) {
-                // separable weights: tap (row r, column q) has weight
-                // wa[r] * wb[q]; rows iu, ju and columns iv, jv relative to
-                // the window origin lie in 0..2 (ju = iu at the chart edge)
-                const int ri = iu - ou, rj = ju - ou, ci = iv - ov, cj = jv - ov;
-                float A[3], Bw[3];
-                window_weights(1.f - fu, fu, ri, rj, A);
-                window_weights(1.f - fv, fv, ci, cj, Bw);
-                // when no valid lane's taps reach window row (column) 2, its
-                // weights are zero on every lane and the window is 2 x 3 (3 x 2);
-                // not for 4 channels, whose kernel has no registers to spare
-                if constexpr (CM <= 3) {
-                    if (!(lanes_where(rj == 2) & vmask)) {
-                        window_texel_add<2, 3, CM>(A, Bw, vval, lane, vtex_chart, ou, ov, s.h,
-                                                   s.w, CM);
-                        return;
-                    }
-                    if (!(lanes_where(cj == 2) & vmask)) {
-                        window_texel_add<3, 2, CM>(A, Bw, vval, lane, vtex_chart, ou, ov, s.h,
-                                                   s.w, CM);
-                        return;
-                    }
-                }
-                window_texel_add<3, 3, CM>(A, Bw, vval, lane, vtex_chart, ou, ov, s.h, s.w, CM);
-                return;
-            }
-            if (tex_lds) {
-                // merge lanes on the same texel quad before the LDS adds
-                const QuadMerge qm = quad_merge_setup(valid ? row[0] : -1, lane);
-                int lofs[4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) lofs[k] = row[k] >> kES;
-#pragma unroll
-                for (int c = 0; c < CM; ++c) {
-                    if (c >= C) break;
-                    float q[4];
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) q[k] = quad_merge(wt[k] * vval[c], qm);
-#pragma unroll
-                    for (int k = 0; k < 4; ++k)
-                        if (q[k] != 0.f) atomicAdd(acc + lofs[k] + c, q[k]);
-                }
-            }
+            for (int k = 0; k < 4; ++k) lofs[k] = row[k] >> kES;
+            texel_gradients<CM>(vtex, quad_val, b.v_texture_out, pid, C, vis, wt, lofs, fu, fv,
+                                fminf((float)s.h * u, (float)(s.h - 1)),
+                                fminf((float)s.w * v, (float)(s.w - 1)), iu, iv, ju, jv, bilinear,
+                                valid, vmask, s.h, s.w, lane, acc, vtex_chart);
         }
-        if constexpr (CM > 4) {
-            if (ch.ok) {
-                int lofs[4];
-#pragma unroll
-                for (int k = 0; k < 4; ++k) lofs[k] = row[k] >> kES;
-                texel_gradients_wide(
-                    b.v_texture_out, pid, C, vis, wt, lofs, fminf((float)s.h * u, (float)(s.h - 1)),
-                    fminf((float)s.w * v, (float)(s.w - 1)), iu, iv, ju, jv, bilinear, valid,
-                    vmask, hw, s.h, s.w, lane, acc, vtex_chart);
-            }
-            return;
-        }
-        if (tex_lds) {
-            // Flush only the texel rows some valid lane touched.
-            int rlo = 0x7fffffff, rhi = -1;
-            if (valid) {
-                rlo = min(min(row[0], row[1]), min(row[2], row[3]));
-                rhi = max(max(row[0], row[1]), max(row[2], row[3]));
-            }
-            rlo = wave_min(rlo);
-            rhi = wave_max(rhi);
-            // every lane's LDS adds precede these reads in the wave's LDS queue
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            const int n_acc = (rhi >> kES) + C;  // past the last value of the last touched texel
-            for (int k = (rlo >> kES) + lane; k < n_acc; k += kWave) {
-                const float v = acc[k];
-                if (v != 0.f) {
-                    unsafeAtomicAdd(vtex_chart + k, v);
-                    acc[k] = 0.f;
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        }
+    };
+
+    // One list entry (wave-uniform index e, Gaussian g with record s).
+    auto entry = [&](const int e, const int g, const Splat& s) {
+        // The pair math and the taps run for every lane: they are finite for
+        // any pixel ray, and tap offsets stay inside the chart.  A lane that
+        // does not contribute keeps T and vT and gets zero seeds (vis, valpha,
+        // vt, vu, vv), so every gradient value below is zero for it without a
+        // branch or per-value selects.
+        const Pair p = pair_eval(s, pr, use_blur, PRECISE && a.precise_edge);
+        const bool valid = e <= last_e && !p.skip;
+        const uint64_t vmask = lanes_where(e <= last_e) & ~skip_lanes(p);
+        if (vmask == 0) return;
+
+        // Transmittance before this Gaussian (1 - alpha >= 0.01) and the texel taps.
+        const Chart ch = chart_of<TB>(a.texture, s, C, a.num_texels);
+        // (a reciprocal and a product: about 1.5 ulp per entry, 3e-6 relative
+        // after a thousand)
+        if (valid) T = T * __builtin_amdgcn_rcpf(1.f - p.alpha);
+        const float vis = valid ? p.alpha * T : 0.f;
+        // A chart of one texel (or none) has one value and no uv gradient: its
+        // taps and the six uv sums are left out (a wave-uniform choice; 1600 x
+        // 1200, 1M Gaussians of one texel: 1020 -> 735 us).
+        const bool flat = !ch.ok || s.h * s.w == 1;
+        if (flat) pixels(e, g, s, p, ch, valid, vmask, vis, std::true_type{});
+        else pixels(e, g, s, p, ch, valid, vmask, vis, std::false_type{});
     };
 
     // Entry order: back to front over [r0, e_hi], in 64-entry windows aligned
@@ -610,43 +587,44 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
     // culled entry has alpha < 1/255 at all of them, so it adds nothing).
     const int mword0 = (r0 >> 6) + tile, mentry0 = r0 & ~63;
     const WaveRect rect = wave_rect(inside, j, i);
-    if (a.wave_masks != nullptr) {
-        // The mask words of 64 windows are read at once, lane k holding window
-        // top - k, so windows this wave never composited (long runs of them in
-        // lists the forward culled or passed over) cost no read of their ids.
-        const size_t plane = (size_t)wave * a.mask_plane + mword0;
-        const uint64_t* mplane = a.wave_masks + plane;
-        const GSTEX_CONST uint64_t* mplane_s = as_const_space(a.wave_masks) + plane;
-        const int top = e_hi >= r0 ? ((e_hi & ~63) - mentry0) >> 6 : -1;
-        for (int wt = top; wt >= 0; wt -= 64) {
-            const int wi = wt - lane;
-            const int wb = mentry0 + (wi << 6);
-            const int lo = max(r0 - wb, 0), hi = min(e_hi - wb, 63);
-            bool any = false;
-            if (wi >= 0 && hi >= lo) any = (mplane[wi] & ((~0ull >> (63 - hi)) & (~0ull << lo))) != 0;
-            uint64_t nz = lanes_where(any);
-            while (nz != 0) {
-                const int k = __ffsll((unsigned long long)nz) - 1;
-                nz &= nz - 1;
-                // the word again, through the scalar path: no vector register
-                // holds it while the entries are processed
-                const int base = mentry0 + ((wt - k) << 6);
-                const Window w = window_candidates<false>(a, base, r0, e_hi, rect, lane, false);
-                uint64_t m = mplane_s[wt - k] & w.in_range;
-                while (m != 0) {
-                    const int bit = 63 - __builtin_clzll(m);
-                    m &= ~(1ull << bit);
-                    const int g = __builtin_amdgcn_readlane(w.gid, bit);
-                    entry(base + bit, g, splat_record(a, g));
-                }
+    const bool masked = a.wave_masks != nullptr;
+    // The mask words of 64 windows are read at once, lane k holding window
+    // top - k, so windows this wave never composited (long runs of them in
+    // lists the forward culled or passed over) cost no read of their ids.
+    const size_t plane = masked ? (size_t)wave * a.mask_plane + mword0 : 0;
+    const uint64_t* mplane = a.wave_masks + plane;
+    const GSTEX_CONST uint64_t* mplane_s = as_const_space(a.wave_masks) + plane;
+    // windows still to visit: without masks window `next` and those below it;
+    // with masks those of the bits nz among next - 63 .. next, then the rest
+    int next = e_hi >= r0 ? ((e_hi & ~63) - mentry0) >> 6 : -1;
+    uint64_t nz = 0;
+    int block = next;  // the top window of the words behind nz
+    for (;;) {
+        int wi;
+        if (masked) {
+            while (nz == 0 && next >= 0) {
+                block = next;
+                next -= 64;
+                const int k = block - lane, wb = mentry0 + (k << 6);
+                const int lo = max(r0 - wb, 0), hi = min(e_hi - wb, 63);
+                bool any = false;
+                if (k >= 0 && hi >= lo)
+                    any = (mplane[k] & ((~0ull >> (63 - hi)) & (~0ull << lo))) != 0;
+                nz = lanes_where(any);
             }
+            if (nz == 0) break;
+            wi = block - (__ffsll((unsigned long long)nz) - 1);
+            nz &= nz - 1;
+        } else {
+            if (next < 0) break;
+            wi = next--;
         }
-        return;
-    }
-    for (int base = e_hi >= r0 ? (e_hi & ~63) : mentry0 - 64; base >= mentry0; base -= 64) {
+        const int base = mentry0 + (wi << 6);
         const Window w = window_candidates<GENERAL>(a, base, r0, e_hi, rect, lane,
-                                                    a.boxes != nullptr, use_blur);
-        uint64_t m = w.cand;
+                                                    !masked && a.boxes != nullptr, use_blur);
+        // (the mask word again, through the scalar path: no vector register
+        // holds it while the entries are processed)
+        uint64_t m = masked ? mplane_s[wi] & w.in_range : w.cand;
         while (m != 0) {
             const int bit = 63 - __builtin_clzll(m);
             m &= ~(1ull << bit);
@@ -665,7 +643,7 @@ __device__ __forceinline__ float* zeroed_tex_acc(float (&tex_acc)[256 / kWave][k
     return acc;
 }
 
-constexpr int bwd_waves_per_eu(int cm, int mode) { return cm > 4 ? 4 : mode == 0 ? 5 : 1; }
+constexpr int bwd_waves_per_eu(int cm, int mode) { return cm <= 4 && mode == 0 ? 5 : 4; }
 
 template <int CM, int MODE, bool TB>
 __global__ __launch_bounds__(256)

@@ -368,6 +368,26 @@ __device__ __forceinline__ void chart_taps_ij(const Splat& s, const Chart& ch, f
     off[3] = off[2] + dv;
 }
 
+// The weights alone (wii, wij, wji, wjj), as chart_taps_ij forms them.
+__device__ __forceinline__ void tap_weights(const Splat& s, float u, float v, bool bilinear,
+                                            float (&wt)[4]) {
+    const float fu = __builtin_amdgcn_fractf((float)s.h * u);
+    const float fv = __builtin_amdgcn_fractf((float)s.w * v);
+    const float wii = (1.f - fu) * (1.f - fv), wij = (1.f - fu) * fv, wji = fu * (1.f - fv),
+                wjj = fu * fv;
+    wt[0] = wii;
+    wt[1] = wij;
+    wt[2] = wji;
+    wt[3] = wjj;
+    if (!bilinear) {
+        const float top = fmaxf(fmaxf(wii, wij), fmaxf(wji, wjj));
+        wt[0] = wii == top ? 1.f : 0.f;
+        wt[1] = wii != top && wij == top ? 1.f : 0.f;
+        wt[2] = wii != top && wij != top && wji == top ? 1.f : 0.f;
+        wt[3] = wii != top && wij != top && wji != top ? 1.f : 0.f;
+    }
+}
+
 __device__ __forceinline__ void chart_taps(const Splat& s, const Chart& ch, float u, float v,
                                            bool bilinear, float wt[4], int off[4], float& fu,
                                            float& fv) {
@@ -558,6 +578,27 @@ __device__ __forceinline__ int rs_slot(int lane) {
 template <int M>
 __device__ __forceinline__ float quad_lane(float v) {
     return dpp<M * 0x55>(v);
+}
+
+// The layout's values: lane j of a quad gets value j (of C <= 4; 0 past them)
+// of each of the quad's four pixels.
+template <int C>
+__device__ __forceinline__ void quad_transpose(const float (&v)[C], int lane, float (&out)[4]) {
+    const int j = lane & 3;
+    auto of = [&](auto lane_m) {
+        constexpr int M = decltype(lane_m)::value;
+        float r = 0.f;
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const float t = quad_lane<M>(v[c]);
+            r = j == c ? t : r;
+        }
+        return r;
+    };
+    out[0] = of(std::integral_constant<int, 0>{});
+    out[1] = of(std::integral_constant<int, 1>{});
+    out[2] = of(std::integral_constant<int, 2>{});
+    out[3] = of(std::integral_constant<int, 3>{});
 }
 
 // Bilinear weight of texel row (column) c at position p along it, both

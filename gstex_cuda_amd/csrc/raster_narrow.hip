@@ -721,16 +721,16 @@ __global__ __launch_bounds__(256) void k_raster_backward_narrow(RasterArgs a, Bw
         gr[G_P22] = vl2 * p.l2;
         gr[G_U1] = vu * p.l1;
         gr[G_U2] = vu * p.l2;
-        gr[G_V1] = vv * p.l1;
-        gr[G_V2] = vv * p.l2;
+        ge[G_V1 - 16] = vv * p.l1;
+        ge[G_V2 - 16] = vv * p.l2;
         gr[G_VL1] = vl1;
         gr[G_VL2] = vl2;
-        gr[G_VU] = vu;
-        gr[G_VV] = vv;
-        ge[G_VNUM - 16] = vnum;
-        ge[G_AX3X + 0 - 16] = vden * pr.r.x + vis * vn.x;
-        ge[G_AX3X + 1 - 16] = vden * pr.r.y + vis * vn.y;
-        ge[G_AX3X + 2 - 16] = vden * pr.r.z + vis * vn.z;
+        ge[G_VU - 16] = vu;
+        ge[G_VV - 16] = vv;
+        gr[G_VNUM] = vnum;
+        gr[G_AX3X + 0] = vden * pr.r.x + vis * vn.x;
+        gr[G_AX3X + 1] = vden * pr.r.y + vis * vn.y;
+        gr[G_AX3X + 2] = vden * pr.r.z + vis * vn.z;
         if constexpr (BLUR) {
             const float vsb = p.blur_sel ? -s.opac * p.Gb * valpha : 0.f;
             ge[4] = 2.0f * vsb * (s.pix_x - pr.px);

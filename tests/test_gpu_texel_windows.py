@@ -102,3 +102,26 @@ def test_wide_gradients_at_chart_edges(oracle, channels, settings, bw):
     ok, l2, frac = grad_close(np_(gg["v_texture"]), og["v_texture"])
     log("wide edges", channels, settings, bw, "relL2 %.2e" % l2, "frac %.4f" % frac)
     assert ok, (l2, frac)
+
+
+# 8x8 tiles: up to four channels on 16x16 tiles take the small-grid kernels here
+@pytest.mark.parametrize("channels,settings", [(1, 0), (2, 0), (3, 0), (4, 0), (3, 1 << 2),
+                                               (4, 1 << 2), (3, 1 << 9), (3, 1 << 10)])
+def test_gradients_at_chart_edges(oracle, channels, settings):
+    s = _scene(20 + channels, channels, 8)
+    settings |= 1 << 8
+    b = project_and_bin(s, 8)
+    g, _ = gpu_forward(s, b["ids"], b["bins"], settings=settings, bw=8)
+    sc = oracle_with(oracle, s, b["ids"], b["bins"], settings=settings, bw=8)
+    o = oracle.texture_forward(sc, "f64")
+    grads = random_grads(np.random.default_rng(2), s.img_h, s.img_w, channels, 1e-3)
+    gg = gpu_backward(s, b["ids"], b["bins"], g, grads, settings=settings, bw=8)
+    og = oracle.texture_backward(sc, o, grads["img"], grads["depth"], grads["reg"],
+                                 grads["alpha"], grads["tex"], grads["normal"], "f64")
+    for k in ("v_texture", "v_uv0", "v_umap", "v_vmap", "v_colors"):
+        ok, l2, frac = grad_close(np_(gg[k]), og[k])
+        log("edges", channels, settings, k, "relL2 %.2e" % l2, "frac %.4f" % frac)
+        assert ok, (k, l2, frac)
+    flat = s.texture_dims[:, 0] * s.texture_dims[:, 1] == 1
+    for k in ("v_uv0", "v_umap", "v_vmap"):  # one texel: no uv gradient at all
+        assert not np_(gg[k])[flat].any(), k
