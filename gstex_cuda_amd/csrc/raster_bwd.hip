@@ -406,7 +406,8 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
                 } else {
                     for (int c = 0; c < C; ++c) d0 = fmaf(chart_texel<TB>(ch, c * E), cot[c], d0);
                 }
-                vvis += (wt[0] * d0 + wt[1] * d0) + (wt[2] * d0 + wt[3] * d0);
+                // rounded as the general case's sum: vvis - vT cancels
+                vvis += fmaf(wt[1], d0, wt[0] * d0) + fmaf(wt[3], d0, wt[2] * d0);
             } else {
                 float D[4] = {0.f, 0.f, 0.f, 0.f};
                 if constexpr (CM <= 4) {
@@ -444,7 +445,7 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
                             for (int k = 0; k < 4; ++k) D[k] = fmaf(tv[k][c], v4[c], D[k]);
                     }
                 }
-                vvis += (wt[0] * D[0] + wt[1] * D[1]) + (wt[2] * D[2] + wt[3] * D[3]);
+                vvis += fmaf(wt[1], D[1], wt[0] * D[0]) + fmaf(wt[3], D[3], wt[2] * D[2]);
                 if (bilinear && prop_uv) {
                     vu = vis * (float)s.h * ((1.f - fv) * (D[2] - D[0]) + fv * (D[3] - D[1]));
                     vv = vis * (float)s.w * ((1.f - fu) * (D[1] - D[0]) + fu * (D[3] - D[2]));
