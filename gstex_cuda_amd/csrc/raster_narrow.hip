@@ -664,9 +664,11 @@ __global__ __launch_bounds__(256) void k_raster_backward_narrow(RasterArgs a, Bw
 #pragma unroll
             for (int k = 0; k < 4; ++k) D[k] = fmaf(tv[k][c], vtex[c], D[k]);
         float vvis = dot3(s.rgb, vo) + dot3(s.a3, vn);
-        vvis += (wt[0] * D[0] + wt[1] * D[1]) + (wt[2] * D[2] + wt[3] * D[3]);
+        // (every fused product below is the one the 8x8 kernel forms: several of
+        // these terms cancel, and optimisers divide by a gradient's size)
+        vvis += fmaf(wt[1], D[1], wt[0] * D[0]) + fmaf(wt[3], D[3], wt[2] * D[2]);
         const float dval = p.t;
-        const float vw = (dval * dval * S0 - 2.f * dval * S1 + S2) * vreg;
+        const float vw = (fmaf(S0, dval * dval, -(2.f * dval * S1)) + S2) * vreg;
 
         // the transmittance and its cotangent through the four entries
         float A[kSlots], V[kSlots], W[kSlots];
@@ -690,15 +692,15 @@ __global__ __launch_bounds__(256) void k_raster_backward_narrow(RasterArgs a, Bw
         const float vis = valid ? p.alpha * my_T : 0.f;
         float vu = 0.f, vv = 0.f;
         if (prop_uv) {
-            vu = vis * (float)s.h * ((1.f - fv) * (D[2] - D[0]) + fv * (D[3] - D[1]));
-            vv = vis * (float)s.w * ((1.f - fu) * (D[1] - D[0]) + fu * (D[3] - D[2]));
+            vu = vis * (float)s.h * fmaf(1.f - fv, D[2] - D[0], fv * (D[3] - D[1]));
+            vv = vis * (float)s.w * fmaf(1.f - fu, D[1] - D[0], fu * (D[3] - D[2]));
         }
         if (!valid) vu = vv = 0.f;  // NaN-safe zero seeds
-        const float vd_val = 2.f * (vis * dval * S0 - vis * S1) * vreg;
-        float valpha = my_T * (vvis - my_vT) + vw * my_T;
+        const float vd_val = 2.f * fmaf(S0, vis * dval, -(vis * S1)) * vreg;
+        float valpha = fmaf(vw, my_T, my_T * (vvis - my_vT));
         valpha = valid ? valpha : 0.f;
         const float vtview = (e == dfin && dfin != -1) ? vdep : 0.f;
-        float vt = vd_val + pr.view_depth * vtview;
+        float vt = fmaf(pr.view_depth, vtview, vd_val);
         vt = valid ? vt : 0.f;
 
         float gr[16], ge[BLUR ? 6 : 4];
@@ -709,9 +711,12 @@ __global__ __launch_bounds__(256) void k_raster_backward_narrow(RasterArgs a, Bw
         const float vsigma = p.blur_sel ? 0.f : -s.opac * p.G * valpha;
         const float vl1 = vsigma * s.iq1 * p.l1;
         const float vl2 = vsigma * s.iq2 * p.l2;
-        const V3 vdelta = v3(vl1 * s.a1.x + vl2 * s.a2.x + s.umap.x * vu + s.vmap.x * vv,
-                             vl1 * s.a1.y + vl2 * s.a2.y + s.umap.y * vu + s.vmap.y * vv,
-                             vl1 * s.a1.z + vl2 * s.a2.z + s.umap.z * vu + s.vmap.z * vv);
+        auto vd = [&](float a1, float a2, float um, float vm) {
+            return fmaf(vm, vv, fmaf(um, vu, fmaf(vl1, a1, vl2 * a2)));
+        };
+        const V3 vdelta = v3(vd(s.a1.x, s.a2.x, s.umap.x, s.vmap.x),
+                             vd(s.a1.y, s.a2.y, s.umap.y, s.vmap.y),
+                             vd(s.a1.z, s.a2.z, s.umap.z, s.vmap.z));
         vt += dot3(vdelta, pr.r);
         const float vnum = vt * __builtin_amdgcn_rcpf(p.den);
         const float vden = -vnum * p.t;
@@ -728,9 +733,9 @@ __global__ __launch_bounds__(256) void k_raster_backward_narrow(RasterArgs a, Bw
         ge[G_VU - 16] = vu;
         ge[G_VV - 16] = vv;
         gr[G_VNUM] = vnum;
-        gr[G_AX3X + 0] = vden * pr.r.x + vis * vn.x;
-        gr[G_AX3X + 1] = vden * pr.r.y + vis * vn.y;
-        gr[G_AX3X + 2] = vden * pr.r.z + vis * vn.z;
+        gr[G_AX3X + 0] = fmaf(vis, vn.x, vden * pr.r.x);
+        gr[G_AX3X + 1] = fmaf(vis, vn.y, vden * pr.r.y);
+        gr[G_AX3X + 2] = fmaf(vis, vn.z, vden * pr.r.z);
         if constexpr (BLUR) {
             const float vsb = p.blur_sel ? -s.opac * p.Gb * valpha : 0.f;
             ge[4] = 2.0f * vsb * (s.pix_x - pr.px);
