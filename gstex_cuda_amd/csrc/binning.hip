@@ -1331,13 +1331,24 @@ __global__ __launch_bounds__(256) void k_bin_prepare(
 }
 
 // offs[p] = sum of w[order[q]] over q < p (w = info.x), and *total = the sum over
-// every p, in one launch: tiles of kWrScanTile positions, 16 consecutive per
+// every p, in one launch: tiles of 256 PER positions, PER consecutive per
 // thread, each tile adding the sum of the tiles before it by a decoupled
 // look-back (ticket order, as in the one-sweep sort).  states holds one
 // look-back state per tile, then the ticket and error words, all zeroed.
 // rec[p] = (offs[p], order[p], its rectangle corner, its rectangle width):
 // what the emission needs of position p, in one 16-byte read.
+// Bound by the latency of its gathers with few tiles, by the tickets and the
+// look-back with many.  16 positions a thread took 14 us for 20k Gaussians, 4 take
+// 5; 16, 8 and 4 take 17, 10 and 10 for 200k, 21, 16 and 20 for 500k, 32, 32 and
+// 38 for 1M, 112, 100 and 110 for 3M.
+constexpr int kPosScanSmallN = 200000;
+static int pos_scan_per(int n) { return n <= kPosScanSmallN ? 4 : 8; }
+static int pos_scan_tiles(int n) {
+    const int tile = 256 * pos_scan_per(n);
+    return (int)(((long long)n + tile - 1) / tile);
+}
 
+template <int PER>
 __global__ __launch_bounds__(256) void k_scan_written(int n, const uint32_t* __restrict__ order,
                                                       const uint4* __restrict__ info,
                                                       uint32_t* __restrict__ offs,
@@ -1347,16 +1358,30 @@ __global__ __launch_bounds__(256) void k_scan_written(int n, const uint32_t* __r
     __shared__ uint32_t lds[256 / kWave];
     __shared__ uint32_t s_blk, s_before;
     uint32_t* const ticket = (uint32_t*)(states + tiles);
+    constexpr int kTile = 256 * PER;
     const int tid = threadIdx.x;
     if (tid == 0) s_blk = atomicAdd(ticket, 1u);
     __syncthreads();
     const int blk = (int)s_blk;
-    const size_t base = (size_t)blk * kWrScanTile + (size_t)tid * kWrScanPer;
-    uint32_t v[kWrScanPer], gs[kWrScanPer], xys[kWrScanPer], wds[kWrScanPer];
+    const size_t base = (size_t)blk * kTile + (size_t)tid * PER;
+    const bool full = base + PER <= (size_t)n;
+    uint32_t v[PER], gs[PER], xys[PER], wds[PER];
+    if (full) {  // order and offs are 16-byte aligned parts of the workspace
+#pragma unroll
+        for (int q = 0; q < PER; q += 4) {
+            const uint4 t = *reinterpret_cast<const uint4*>(order + base + q);
+            gs[q] = t.x;
+            gs[q + 1] = t.y;
+            gs[q + 2] = t.z;
+            gs[q + 3] = t.w;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < PER; ++j) gs[j] = base + j < (size_t)n ? order[base + j] : 0u;
+    }
     uint32_t sum = 0;
 #pragma unroll
-    for (int j = 0; j < kWrScanPer; ++j) {
-        gs[j] = base + j < (size_t)n ? order[base + j] : 0u;
+    for (int j = 0; j < PER; ++j) {
         const uint4 f = base + j < (size_t)n ? info[gs[j]] : make_uint4(0u, 0u, 1u, 0u);
         v[j] = f.x;
         xys[j] = f.y;
@@ -1375,18 +1400,27 @@ __global__ __launch_bounds__(256) void k_scan_written(int n, const uint32_t* __r
         }
         if (tid == 0) {
             s_before = (uint32_t)before;
-            if ((size_t)(blk + 1) * kWrScanTile >= (size_t)n) *total = (uint32_t)(before + tot);
+            if ((size_t)(blk + 1) * kTile >= (size_t)n) *total = (uint32_t)(before + tot);
         }
     }
     __syncthreads();
     uint32_t run = s_before + excl;
+    uint32_t at[PER];
 #pragma unroll
-    for (int j = 0; j < kWrScanPer; ++j) {
-        if (base + j < (size_t)n) {
-            offs[base + j] = run;
-            rec[base + j] = make_uint4(run, gs[j], xys[j], wds[j]);
-        }
+    for (int j = 0; j < PER; ++j) {
+        at[j] = run;
+        if (base + j < (size_t)n) rec[base + j] = make_uint4(run, gs[j], xys[j], wds[j]);
         run += v[j];
+    }
+    if (full) {
+#pragma unroll
+        for (int q = 0; q < PER; q += 4)
+            *reinterpret_cast<uint4*>(offs + base + q) =
+                make_uint4(at[q], at[q + 1], at[q + 2], at[q + 3]);
+    } else {
+#pragma unroll
+        for (int j = 0; j < PER; ++j)
+            if (base + j < (size_t)n) offs[base + j] = at[j];
     }
 }
 
@@ -1759,7 +1793,7 @@ static DepthWs depth_ws(int n, void* base) {
     d.info = (uint4*)take(16 * (size_t)n);
     d.rec = (uint4*)take(16 * (size_t)n);
     d.offs = (uint32_t*)take(4 * (size_t)n + 8);
-    d.states = (uint64_t*)take(8 * ((size_t)wr_scan_tiles(n) + 1));
+    d.states = (uint64_t*)take(8 * ((size_t)pos_scan_tiles(n) + 1));
     d.rws_bytes = up256(radix_workspace_bytes<uint32_t>(n));
     d.rws = take(d.rws_bytes);
     d.total = at;
@@ -1814,7 +1848,7 @@ static hipError_t bin_depth_phase(int n, const float* centers, const float* exte
                                   const float* depths, const int* counts, int tiles_x,
                                   int tiles_y, int bw, int* tile_bins, const DepthWs& d,
                                   int m_exact, hipStream_t s) {
-    const int gn = (n + 255) / 256, st = wr_scan_tiles(n);
+    const int gn = (n + 255) / 256, st = pos_scan_tiles(n);
     uint32_t* total = d.offs + n;  // entries written by Gaussians
     k_bin_prepare<<<gn, 256, 0, s>>>(n, centers, extents, depths, counts, tiles_x, tiles_y, bw,
                                      d.dkey, d.ord, d.info, tile_bins, 2 * tiles_x * tiles_y,
@@ -1823,7 +1857,10 @@ static hipError_t bin_depth_phase(int n, const float* centers, const float* exte
     if (e != hipSuccess) return e;
     e = radix_sort_pairs<uint32_t>(n, d.dkey, d.ord, d.dkey2, d.ord2, 32, d.rws, d.rws_bytes, s);
     if (e != hipSuccess) return e;
-    k_scan_written<<<st, 256, 0, s>>>(n, d.ord2, d.info, d.offs, d.rec, total, d.states, st);
+    if (pos_scan_per(n) == 4)
+        k_scan_written<4><<<st, 256, 0, s>>>(n, d.ord2, d.info, d.offs, d.rec, total, d.states, st);
+    else
+        k_scan_written<8><<<st, 256, 0, s>>>(n, d.ord2, d.info, d.offs, d.rec, total, d.states, st);
     return hipGetLastError();
 }
 
