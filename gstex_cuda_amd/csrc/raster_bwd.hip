@@ -100,6 +100,9 @@ __device__ __forceinline__ void cotangents4(const float* src, int C, int cb, flo
 //   lds     charts of up to kTexAccFloats values: lanes on one quad merged,
 //           then LDS adds and a flush
 //   direct  one atomic per tap and channel
+// The merged sums weigh lanes and texels that a pixel has no part in by zero, so
+// they need finite cotangents.  With OWN (waves of four and more channels that
+// hold others) a lane adds to its own taps alone, on the lds and direct routes.
 // Bound by instruction issue.  A pass over 50k Gaussians at 800 x 600 with 8
 // channels took 4.9 ms with per-lane LDS or global atomics, which serialise
 // where the lanes of a wave meet on one texel, 1.46 ms with these routes; wave
@@ -107,7 +110,7 @@ __device__ __forceinline__ void cotangents4(const float* src, int C, int cb, flo
 // blur), the matrix instructions 700.  Four channels, 50k Gaussians at 1600 x 1200: 774 us by
 // wave reductions, 658; three or fewer gain nothing (985 us either way at 1080p,
 // 500k Gaussians).
-template <int CM>
+template <int CM, bool OWN>
 __device__ __forceinline__ void texel_gradients(
     const float (&vtex)[CM <= 4 ? CM : 1], const float (&quad_val)[4], const float* v_texture_out,
     int pid, int C, float vis, const float (&wt)[4], const int (&lofs)[4], float fu, float fv,
@@ -128,10 +131,10 @@ __device__ __forceinline__ void texel_gradients(
     // when some valid lane lies below it
     const int au = __builtin_amdgcn_readlane(iu, first);
     const int av = __builtin_amdgcn_readlane(iv, first);
-    const bool quad = !((lanes_where(iu != au) | lanes_where(iv != av)) & vmask);
+    const bool quad = !OWN && !((lanes_where(iu != au) | lanes_where(iv != av)) & vmask);
     int ou = au, ov = av;
     bool window = false;
-    if (!quad && bilinear) {
+    if (!OWN && !quad && bilinear) {
         ou = au - ((lanes_where(iu < au) & vmask) ? 1 : 0);
         ov = av - ((lanes_where(iv < av) & vmask) ? 1 : 0);
         window = !(lanes_where(((uint32_t)(iu - ou) | (uint32_t)(iv - ov)) > 1u) & vmask);
@@ -250,6 +253,7 @@ __device__ __forceinline__ void texel_gradients(
         for (int c = 0; c < G; ++c)
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
+                if (OWN && !valid) continue;
                 const float add = wt[k] * (vis * vtex[CM <= 4 ? c : 0]);
                 if (add != 0.f) unsafeAtomicAdd(vtex_chart + lofs[k] + c, add);
             }
@@ -263,7 +267,10 @@ __device__ __forceinline__ void texel_gradients(
         for (int c = 0; c < G; ++c) {
             float q[4];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) q[k] = quad_merge(wt[k] * (vis * v[c]), qm);
+            for (int k = 0; k < 4; ++k) {
+                if constexpr (OWN) q[k] = valid ? wt[k] * (vis * v[c]) : 0.f;
+                else q[k] = quad_merge(wt[k] * (vis * v[c]), qm);
+            }
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 if (q[k] == 0.f || cb + c >= C) continue;
@@ -293,11 +300,32 @@ __device__ __forceinline__ void texel_gradients(
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
 }
 
+// Whether every texture cotangent that the lanes of a wave read is finite (a
+// lane outside the image reads pixel 0's; see raster_backward_wave).
+__device__ __forceinline__ bool cotangents_finite(const RasterArgs& a, const BwdIn& b,
+                                                  const int tile, const int wave, const int C) {
+    const int ty = tile / a.tiles_x, tx = tile - ty * a.tiles_x;
+    int lx, ly;
+    bool in_tile;
+    lane_pixel(a.bw, wave * kWave + (threadIdx.x & (kWave - 1)), lx, ly, in_tile);
+    const int j = tx * a.bw + lx, i = ty * a.bw + ly;
+    const bool inside = in_tile && i < a.img_h && j < a.img_w;
+    const float* const cot = b.v_texture_out + (size_t)(inside ? i * a.img_w + j : 0) * C;
+    bool finite = true;
+    for (int cb = 0; cb < C; cb += 4) {
+        float v[4];
+        cotangents4(cot, C, cb, v);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) finite = finite && fabsf(v[c]) < INFINITY;
+    }
+    return lanes_where(!finite) == 0;
+}
+
 // raster_backward_wave runs one wave's share of a tile (wave `wave` of the
 // tile, as in the forward); `acc` is this hardware wave's LDS texel
-// accumulator, zero on entry and left zero.
-template <int CM, int MODE, bool TB>
-__device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const BwdIn& b,
+// accumulator, zero on entry and left zero.  OWN: see texel_gradients.
+template <int CM, int MODE, bool TB, bool OWN>
+__device__ __forceinline__ void raster_backward_entries(const RasterArgs& a, const BwdIn& b,
                                                      const int tile, const int wave,
                                                      float* const acc) {
     constexpr bool GENERAL = MODE == 1, PRECISE = MODE != 0;
@@ -355,7 +383,7 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
              b.v_alpha[pid];
     }
     float quad_val[4] = {0.f, 0.f, 0.f, 0.f};
-    if constexpr (CM == 4) quad_transpose(vtex, lane, quad_val);
+    if constexpr (CM == 4 && !OWN) quad_transpose(vtex, lane, quad_val);
     int r0, r1;
     tile_range(a, tile, r0, r1);
     // Entries past the wave's last contributing index are dead for every lane.
@@ -540,6 +568,10 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
 #pragma unroll
                     for (int c = 0; c < G; ++c) vals[c] *= vis * wsum;
                 }
+                if constexpr (OWN) {
+#pragma unroll
+                    for (int c = 0; c < G; ++c) vals[c] = valid ? vals[c] : 0.f;
+                }
                 const float tot = wave_reduce_scatter(vals, lane);
                 if (code < 64 && cb + code < C && tot != 0.f)
                     unsafeAtomicAdd(vtex_chart + cb + code, tot);
@@ -548,10 +580,10 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
             int lofs[4];
 #pragma unroll
             for (int k = 0; k < 4; ++k) lofs[k] = row[k] >> kES;
-            texel_gradients<CM>(vtex, quad_val, b.v_texture_out, pid, C, vis, wt, lofs, fu, fv,
-                                fminf((float)s.h * u, (float)(s.h - 1)),
-                                fminf((float)s.w * v, (float)(s.w - 1)), iu, iv, ju, jv, bilinear,
-                                valid, vmask, s.h, s.w, lane, acc, vtex_chart);
+            texel_gradients<CM, OWN>(
+                vtex, quad_val, b.v_texture_out, pid, C, vis, wt, lofs, fu, fv,
+                fminf((float)s.h * u, (float)(s.h - 1)), fminf((float)s.w * v, (float)(s.w - 1)),
+                iu, iv, ju, jv, bilinear, valid, vmask, s.h, s.w, lane, acc, vtex_chart);
         }
     };
 
@@ -633,6 +665,21 @@ __device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const 
             entry(base + bit, g, splat_record(a, g));
         }
     }
+}
+
+template <int CM, int MODE, bool TB>
+__device__ __forceinline__ void raster_backward_wave(const RasterArgs& a, const BwdIn& b,
+                                                     const int tile, const int wave,
+                                                     float* const acc) {
+    // (two copies of the walk: a choice within one costs the kernels for four
+    // and more channels 1 to 12 percent, in registers)
+    if constexpr (CM >= 4) {
+        if (!cotangents_finite(a, b, tile, wave, CM <= 4 ? CM : a.channels)) {
+            raster_backward_entries<CM, MODE, TB, true>(a, b, tile, wave, acc);
+            return;
+        }
+    }
+    raster_backward_entries<CM, MODE, TB, false>(a, b, tile, wave, acc);
 }
 
 // Wave-private texel-gradient accumulator (one chart at a time), zeroed once
