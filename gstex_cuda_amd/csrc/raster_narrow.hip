@@ -616,6 +616,12 @@ __global__ __launch_bounds__(256) void k_raster_backward_narrow(RasterArgs a, Bw
         vT = a.background[0] * vo.x + a.background[1] * vo.y + a.background[2] * vo.z -
              b.v_alpha[pid];
     }
+    // pixels with a texture cotangent that is not finite: a window's sums weigh
+    // texels which they do not sample by zero
+    bool finite = true;
+#pragma unroll
+    for (int c = 0; c < CM; ++c) finite = finite && fabsf(vtex[c]) < INFINITY;
+    const uint64_t bad = lanes_where(!finite);
     for (int k = threadIdx.x; k < kTexPool; k += 256) s_pool[k] = 0.f;
     int r0, r1;
     tile_range(a, tile, r0, r1);
@@ -758,7 +764,8 @@ __global__ __launch_bounds__(256) void k_raster_backward_narrow(RasterArgs a, Bw
         // Texel gradients.  A row whose valid lanes' taps lie in one 3x3
         // texel window (2x2 where that holds for every such row) inside its
         // entry's 4x4 window reduces the values of its texels and adds them
-        // there; the lanes of other rows add their taps to memory.
+        // there; the lanes of other rows, and of rows with a pixel of `bad`, add
+        // their own taps.
         const uint64_t okmask = vmask & lanes_where(ok);
         if (okmask == 0) return;
         const bool part = lane_of(okmask);
@@ -774,7 +781,7 @@ __global__ __launch_bounds__(256) void k_raster_backward_narrow(RasterArgs a, Bw
         const int au = __shfl((int)(anchor >> 32), lane & 48), av = __shfl((int)anchor, lane & 48);
         const int ri = iu - ou, rj = ju - ou, ci = iv - ov, cj = jv - ov;
         const uint64_t far =
-            okmask & (lanes_where(((uint32_t)ri | (uint32_t)ci) > 1u) |
+            okmask & (bad | lanes_where(((uint32_t)ri | (uint32_t)ci) > 1u) |
                       lanes_where((uint32_t)(iu - au) >= (uint32_t)kTexWin) |
                       lanes_where((uint32_t)(ju - au) >= (uint32_t)kTexWin) |
                       lanes_where((uint32_t)(iv - av) >= (uint32_t)kTexWin) |

@@ -1,6 +1,7 @@
 """A pixel with a cotangent that is not finite gives such texel gradients only to
 the texels it samples: on images whose sides are not multiples of the tile, at
-pixel (0, 0) and inside, on the routes of four and more channels."""
+pixel (0, 0) and inside, on the routes of four and more channels and in the
+kernels for small tile grids."""
 import numpy as np
 import pytest
 
@@ -43,3 +44,9 @@ def _check(oracle, channels, bw, settings, bad, pixels, seed):
 def test_wide_channels(oracle, channels, bw, settings, bad):
     _check(oracle, channels, bw, settings, bad, [(0, 0)], channels + bw)
     _check(oracle, channels, bw, settings, bad, [(40, 50), (89, 116)], channels + bw)
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+@pytest.mark.parametrize("channels,settings", [(1, 0), (3, 0), (4, 0), (3, 1 << 9)])
+def test_small_grids(oracle, channels, settings, bad):
+    _check(oracle, channels, 16, settings, bad, [(40, 50), (89, 116)], channels + 40)
