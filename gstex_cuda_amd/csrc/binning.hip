@@ -1249,9 +1249,16 @@ hipError_t radix_sort_pairs(int n, const K* keys_in, const uint32_t* vals_in, K*
     // histogram and scan.  Measured at 1080p / 500k: the 500k-key depth sort
     // (245 tiles) 108 -> 78 us, the 11.5M-key tile sort (2805 tiles) 173 -> 197 us.
     if constexpr (sizeof(K) == 4) {
-        // (in place the passes' first write would go to the workspace)
-        if (n <= kRankSortN && start_bit == 0 && end_bit == 32 && keys_in != keys_out &&
-            (vals_in == nullptr || vals_in != vals_out)) {
+        // Its workgroups write while others read, so no output may share memory
+        // with an input; the four passes, the first of which writes to the
+        // workspace, take such calls.
+        auto shared = [n](const void* in, const void* out) {
+            const uintptr_t x = (uintptr_t)in, y = (uintptr_t)out, bytes = 4 * (uintptr_t)n;
+            return in != nullptr && out != nullptr && x < y + bytes && y < x + bytes;
+        };
+        if (n <= kRankSortN && start_bit == 0 && end_bit == 32 && !shared(keys_in, keys_out) &&
+            !shared(keys_in, vals_out) && !shared(vals_in, keys_out) &&
+            !shared(vals_in, vals_out)) {
             k_rank_sort<<<(n + kWave - 1) / kWave, kRankThreads, 0, s>>>(
                 n, (const uint32_t*)keys_in, vals_in, (uint32_t*)keys_out, vals_out);
             return hipGetLastError();

@@ -152,7 +152,10 @@ int gstex_sort_intersects(int num_intersects, int end_bit, const int64_t *isect_
  * texture_sample adjoint use, for callers that sort their own 32-bit keys.
  * Stable ascending radix sort of (uint32 key, uint32 value) pairs over key
  * bits [0, end_bit) (end_bit <= 32; higher key bits are carried, not
- * compared), one launch per 8-bit digit plus one histogram launch. */
+ * compared): one launch for up to 8,192 pairs and all 32 bits, unless an output
+ * shares memory with an input; else one launch per 8-bit digit plus one
+ * histogram launch.  A sort by all 32 bits takes outputs that share memory with
+ * the inputs in any way. */
 size_t gstex_sort_pairs_u32_workspace_size(int n);
 int gstex_sort_pairs_u32(int n, int end_bit, const uint32_t *keys, const uint32_t *values,
                          uint32_t *keys_sorted, uint32_t *values_sorted, void *workspace,
