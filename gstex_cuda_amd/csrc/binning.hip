@@ -174,9 +174,12 @@ __global__ __launch_bounds__(256) void k_map_intersects(
                 int x1, y1;
                 if (wrapped) tile_rect_wrapped(c.x, c.y, e.x, e.y, bw, x0, y0, x1, y1);
                 else tile_rect(c.x, c.y, e.x, e.y, bw, tiles_x, tiles_y, x0, y0, x1, y1);
-                const long long area = (long long)max(x1 - x0, 0) * (long long)max(y1 - y0, 0);
-                k_end = (int)min(area, 0x7fffffffll);
-                w = max(x1 - x0, 1);
+                // (a wrapped rectangle of huge extents is wider than an int holds)
+                const long long top = 0x7fffffffll;
+                const long long cols = min(max((long long)x1 - x0, 0ll), top);
+                const long long rows = min(max((long long)y1 - y0, 0ll), top);
+                k_end = (int)min(cols * rows, top);
+                w = max((int)cols, 1);
             }
             did = (int64_t)__float_as_int(depths[g]);
         }

@@ -1,4 +1,5 @@
-"""The intersect keys of scenes with long runs of Gaussians that count nothing."""
+"""The intersect keys of scenes with long runs of Gaussians that count nothing, and
+of wrapped rectangles wider than a 32-bit integer holds."""
 import numpy as np
 import pytest
 import torch
@@ -52,3 +53,34 @@ def test_zero_run_time():
         times.append(e[0].elapsed_time(e[1]) / 3)
     log("map ms, spread and in one run", times)
     assert times[1] < 4 * times[0] + 1.0
+
+
+@pytest.mark.parametrize("axis", [0, 1, None])
+def test_wrapped_huge_extent(axis):
+    # tile corners saturate at the ends of the 32-bit range; each Gaussian writes
+    # the first tiles of its row-major rectangle, as many as it counts
+    from gstex_cuda_amd import cuda as _C
+
+    lo, nx, ny = -2**31, 20, 13
+    e = np.full((3, 2), 1e12, np.float32)
+    if axis is not None:
+        e[:, 1 - axis] = 12.0  # tiles 5..7
+    c = np.full((3, 2), 100, np.float32)
+    d = np.array([1, 2, 3], np.float32)
+    counts = np.array([5, 40, 3000])
+    cum = np.cumsum(counts).astype(np.int32)
+    keys, ids = _C.map_gaussian_to_intersects(3, int(cum[-1]), to_dev(c), to_dev(e), to_dev(d),
+                                              to_dev(cum), (nx, ny, 1), 16, wrapped=True)
+    x0, x1 = (5, 8) if axis == 1 else (lo, 2**31 - 1)
+    y0, y1 = (5, 8) if axis == 0 else (lo, 2**31 - 1)
+    want_k, want_i = [], []
+    for g in range(3):
+        k = np.arange(counts[g])
+        r, q = k // (x1 - x0), k % (x1 - x0)
+        tile = ((y0 + r) % ny) * nx + (x0 + q) % nx
+        key = (tile.astype(np.int64) << 32) | int(d[g:g + 1].view(np.int32)[0])
+        written = r < y1 - y0
+        want_k.append(np.where(written, key, 0))
+        want_i.append(np.where(written, g, 0))
+    assert np.array_equal(np_(keys), np.concatenate(want_k))
+    assert np.array_equal(np_(ids), np.concatenate(want_i))
