@@ -1126,7 +1126,11 @@ static size_t onesweep_state_words(int n) {
 
 template <typename K>
 size_t radix_workspace_bytes(int n) {
-    const size_t nb = (size_t)sort_blocks(n, sizeof(K));
+    // 64-bit keys: room for every sort of up to n pairs (just below kSortSmallN64 the
+    // tiles are more than at it), so that a workspace sized for the most pairs
+    // does for fewer
+    const int few = sizeof(K) == 8 ? std::min(n, kSortSmallN64 - 1) : n;
+    const size_t nb = (size_t)std::max(sort_blocks(n, sizeof(K)), sort_blocks(few, sizeof(K)));
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t lsd = up(sizeof(uint32_t) * 256 * nb) +
                        up(sizeof(uint64_t) * scan_partials_count((int)(256 * nb)));
