@@ -418,6 +418,10 @@ __device__ __forceinline__ void raster_backward_entries(const RasterArgs& a, con
             gr[G_RGB + 0] = vis * vo.x;
             gr[G_RGB + 1] = vis * vo.y;
             gr[G_RGB + 2] = vis * vo.z;
+            // (the fused products below are written out: several of these terms
+            // cancel and optimisers divide by a gradient's size, so every
+            // instantiation and both kinds of chart round alike, as the kernels
+            // for small tile grids do)
             float vvis = dot3(s.rgb, vo) + dot3(s.a3, vn);
             float vu = 0.f, vv = 0.f;
             // D[k] = sum over channels of vtex[c] * (tap k's texel, channel c).
@@ -434,7 +438,6 @@ __device__ __forceinline__ void raster_backward_entries(const RasterArgs& a, con
                 } else {
                     for (int c = 0; c < C; ++c) d0 = fmaf(chart_texel<TB>(ch, c * E), cot[c], d0);
                 }
-                // rounded as the general case's sum: vvis - vT cancels
                 vvis += fmaf(wt[1], d0, wt[0] * d0) + fmaf(wt[3], d0, wt[2] * d0);
             } else {
                 float D[4] = {0.f, 0.f, 0.f, 0.f};
@@ -475,40 +478,41 @@ __device__ __forceinline__ void raster_backward_entries(const RasterArgs& a, con
                 }
                 vvis += fmaf(wt[1], D[1], wt[0] * D[0]) + fmaf(wt[3], D[3], wt[2] * D[2]);
                 if (bilinear && prop_uv) {
-                    vu = vis * (float)s.h * ((1.f - fv) * (D[2] - D[0]) + fv * (D[3] - D[1]));
-                    vv = vis * (float)s.w * ((1.f - fu) * (D[1] - D[0]) + fu * (D[3] - D[2]));
+                    vu = vis * (float)s.h * fmaf(1.f - fv, D[2] - D[0], fv * (D[3] - D[1]));
+                    vv = vis * (float)s.w * fmaf(1.f - fu, D[1] - D[0], fu * (D[3] - D[2]));
                 }
             }
 
             if (!FLAT && !valid) vu = vv = 0.f;  // NaN-safe zero seeds
             const float dvis = vvis - vT;
-            float valpha = T * dvis;
-            float vTcur = fmaf(p.alpha, dvis, vT);  // alpha vvis + (1 - alpha) vT
             const float t_view = p.t * pr.view_depth;
             const float dval = use_ndc ? (tf * t_view - tf * tn) / ((tf - tn) * t_view) : p.t;
-            const float vd_val = 2.f * (vis * dval * S0 - vis * S1) * vreg;
-            const float vw = (dval * dval * S0 - 2.f * dval * S1 + S2) * vreg;
-            valpha += vw * T;
-            vTcur += vw * p.alpha;
+            const float vd_val = 2.f * fmaf(S0, vis * dval, -(vis * S1)) * vreg;
+            const float vw = (fmaf(S0, dval * dval, -(2.f * dval * S1)) + S2) * vreg;
+            // (two roundings of one sum: each the one its kernels have always formed)
+            float valpha = GENERAL ? fmaf(T, dvis, vw * T) : fmaf(vw, T, T * dvis);
+            // alpha vvis + (1 - alpha) vT, and the distortion's share
+            const float vTcur = fmaf(vw, p.alpha, fmaf(p.alpha, dvis, vT));
             if (valid) vT = vTcur;
             valpha = valid ? valpha : 0.f;
 
             float vt = use_ndc ? 0.f : vd_val;
             float vtview = (e == dfin && dfin != -1) ? vdep : 0.f;
-            if (use_ndc) vtview += (tf * tn) / ((tf - tn) * t_view * t_view) * vd_val;
-            vt += pr.view_depth * vtview;
+            if (use_ndc)
+                vtview = fmaf((tf * tn) / ((tf - tn) * t_view * t_view), vd_val, vtview);
+            vt = fmaf(pr.view_depth, vtview, vt);
             vt = valid ? vt : 0.f;
 
             gr[G_OPAC] = (p.blur_sel ? p.Gb : p.G) * valpha;
             const float vsigma = p.blur_sel ? 0.f : -s.opac * p.G * valpha;
             const float vl1 = vsigma * s.iq1 * p.l1;
             const float vl2 = vsigma * s.iq2 * p.l2;
-            V3 vdelta = v3(vl1 * s.a1.x + vl2 * s.a2.x, vl1 * s.a1.y + vl2 * s.a2.y,
-                           vl1 * s.a1.z + vl2 * s.a2.z);
+            V3 vdelta = v3(fmaf(vl1, s.a1.x, vl2 * s.a2.x), fmaf(vl1, s.a1.y, vl2 * s.a2.y),
+                           fmaf(vl1, s.a1.z, vl2 * s.a2.z));
             if constexpr (!FLAT)
-                vdelta = v3(vdelta.x + s.umap.x * vu + s.vmap.x * vv,
-                            vdelta.y + s.umap.y * vu + s.vmap.y * vv,
-                            vdelta.z + s.umap.z * vu + s.vmap.z * vv);
+                vdelta = v3(fmaf(s.vmap.x, vv, fmaf(s.umap.x, vu, vdelta.x)),
+                            fmaf(s.vmap.y, vv, fmaf(s.umap.y, vu, vdelta.y)),
+                            fmaf(s.vmap.z, vv, fmaf(s.umap.z, vu, vdelta.z)));
             vt += dot3(vdelta, pr.r);
             const float vnum = vt * __builtin_amdgcn_rcpf(p.den);
             const float vden = -vnum * p.t;
@@ -519,9 +523,9 @@ __device__ __forceinline__ void raster_backward_entries(const RasterArgs& a, con
             gr[G_VL1] = vl1;
             gr[G_VL2] = vl2;
             gr[G_VNUM] = vnum;
-            gr[G_AX3X + 0] = vden * pr.r.x + vis * vn.x;
-            gr[G_AX3X + 1] = vden * pr.r.y + vis * vn.y;
-            gr[G_AX3X + 2] = vden * pr.r.z + vis * vn.z;
+            gr[G_AX3X + 0] = fmaf(vis, vn.x, vden * pr.r.x);
+            gr[G_AX3X + 1] = fmaf(vis, vn.y, vden * pr.r.y);
+            gr[G_AX3X + 2] = fmaf(vis, vn.z, vden * pr.r.z);
             if constexpr (!FLAT) {
                 gr[G_U1] = vu * p.l1;
                 gr[G_U2] = vu * p.l2;
