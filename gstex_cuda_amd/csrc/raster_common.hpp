@@ -923,19 +923,32 @@ inline RasterArgs make_raster_args(const RasterCall& c, const float* records) {
 }
 
 // The kernels of raster_narrow.hip take grids of up to kNarrowTiles tiles
-// whose lists hold at most kNarrowForwardIds (kNarrowBackwardIds) entries:
+// whose id buffers hold at most kNarrowForwardIds (kNarrowBackwardIds) entries:
 // there the 8x8 kernels are bound by their longest wave.  With more work the
 // chip fills, and the narrow kernels' instruction count, about twice that of
-// the 8x8 kernels on full waves, decides.  Measured (forward + backward of
-// three channels, 8x8 against narrow): 256 tiles, 66K entries 263 + 431 us
-// against 114 + 193; 920 tiles, 96K 223 + 368 against 112 + 208; 920 tiles,
-// 480K 199 + 383 against 133 + 327; 900 tiles, 405K 186 + 336 against
-// 140 + 335; 1350 tiles, 271K 175 + 303 against 133 + 294; but 1024 tiles,
-// 737K 177 + 375 against 175 + 436, 1900 tiles, 120K 101 + 209 against
-// 113 + 232 and 3600 tiles, 97K 76 + 160 against 113 + 229.
+// the 8x8 kernels on full waves, decides.  (The buffer's size is what the host
+// knows: with a capacity far above the list's length the 8x8 kernels run.)
+// Measured (forward + backward of three channels, 8x8 against narrow): 256
+// tiles, 66K entries 263 + 431 us against 114 + 193; 920 tiles, 96K 223 + 368
+// against 112 + 208; 920 tiles, 480K 199 + 383 against 133 + 327; 900 tiles,
+// 405K 186 + 336 against 140 + 335; 1350 tiles, 271K 175 + 303 against
+// 133 + 294; but 1024 tiles, 737K 177 + 375 against 175 + 436, 1900 tiles, 120K
+// 101 + 209 against 113 + 232 and 3600 tiles, 97K 76 + 160 against 113 + 229.
+// One, two and four channels, the blur and bfloat16 gain as much or more (256 to
+// 1350 tiles: both together 1.2 to 2.3 times as fast).
+//
+// The narrow backward holds a 4x4 texel window of a chart in LDS and four or more
+// whole charts a batch; what exceeds these goes out tap by tap, which costs as
+// the texel values that the lists name: entries times the mean values of a
+// chart.  Up to kNarrowBackwardValues of them it is no slower (charts sized by
+// area, 920 tiles, backward alone: 150K entries of 24 values a chart 366 against
+// 253 us, 70K of 48 462 against 378, 31K of 96 320 against 312); above it 150K of 48
+// 422 against 598, 70K of 96 526 against 675 and, 16x16 texels each, 136K of 768
+// 681 against 1707.
 constexpr int kNarrowTiles = 1400;
 constexpr int kNarrowForwardIds = 600000;
 constexpr int kNarrowBackwardIds = 450000;
+constexpr double kNarrowBackwardValues = 4.5e6;
 bool raster_forward_is_narrow(const RasterArgs& a);
 bool raster_backward_is_narrow(const RasterArgs& a);
 hipError_t raster_forward_narrow(const RasterArgs& a, const FwdOut& o, hipStream_t s);

@@ -993,7 +993,8 @@ bool raster_forward_is_narrow(const RasterArgs& a) {
     return narrow_supported(a) && a.num_ids <= kNarrowForwardIds;
 }
 bool raster_backward_is_narrow(const RasterArgs& a) {
-    return narrow_supported(a) && a.num_ids <= kNarrowBackwardIds;
+    return narrow_supported(a) && a.num_ids <= kNarrowBackwardIds &&
+           (double)a.num_ids * a.channels * a.num_texels <= kNarrowBackwardValues * a.num_points;
 }
 
 template <int CM>
