@@ -11,17 +11,16 @@
 
 namespace gstex {
 
-// Coefficient k of a float32 or bfloat16 (uint16 bits, widened exactly) array.
-__device__ __forceinline__ float coef(const float* c, int k) { return c[k]; }
-__device__ __forceinline__ float coef(const unsigned short* c, int k) {
-    return __uint_as_float((unsigned)c[k] << 16);
-}
-
-// A row of bfloat16 coefficients in 32-bit words (two per word).
-struct Bf16Words {
+// A row of coefficients, float32 or bfloat16 (uint16 bits, two per word, widened
+// exactly), in 32-bit words.
+template <typename CT>
+struct RowWords {
     const uint32_t* w;
 };
-__device__ __forceinline__ float coef(const Bf16Words& c, int k) {
+__device__ __forceinline__ float coef(const RowWords<float>& c, int k) {
+    return __uint_as_float(c.w[k]);
+}
+__device__ __forceinline__ float coef(const RowWords<unsigned short>& c, int k) {
     const uint32_t x = c.w[k >> 1];
     return __uint_as_float((k & 1) ? x & 0xffff0000u : x << 16);
 }
@@ -70,21 +69,30 @@ __device__ __forceinline__ void sh_color(int i, const float* __restrict__ dirs,
 // evaluated up to degree D in float32.
 // With c2w (4 x 4 row-major camera-to-world), dirs holds the means and the
 // direction of Gaussian i is means[i] - c2w[:3, 3] (one float32 subtraction
-// per component).  With staging (rows of whole 32-bit words, 16-byte aligned,
-// and dynamic LDS of 256 rows of row_words | 1 words), the block's coefficient
+// per component).  STAGED (rows of whole 32-bit words, 16-byte aligned, and
+// dynamic LDS of 256 rows of row_words | 1 words): the block's coefficient
 // rows, one contiguous span, come in as 16-byte loads of consecutive addresses
 // and each thread reads its row from LDS (rows padded to an odd word count).
-// Read directly, each of a lane's loads touches 64 cache lines per wave: 3M
-// Gaussians of degree 3 in bfloat16 took 107 us directly, 81 us staged.
-template <int D, typename CT>
+// 3M Gaussians of degree 3 in bfloat16 took 107 us with each coefficient read
+// where it is used, 81 us staged.
+// Other rows (degree 4 above all) are loaded whole into registers first, so that
+// their latency is waited for once, in a kernel of their own: read where used,
+// and in one kernel with the staging, 1M Gaussians of degree 4 took 112 us in
+// float32 and 55 in bfloat16 (the latter 44 before the staging); 69 and 33.
+template <int D, typename CT, bool STAGED>
 __global__ __launch_bounds__(256) void k_sh_forward(int n, int nb, const float* __restrict__ dirs,
                                                     const float* __restrict__ c2w,
                                                     const CT* __restrict__ coeffs,
-                                                    float* __restrict__ colors, bool staged) {
+                                                    float* __restrict__ colors) {
     extern __shared__ uint32_t coef_stage[];
     const int i0 = blockIdx.x * blockDim.x, i = i0 + threadIdx.x;
-    if (!staged) {
-        if (i < n) sh_color<D>(i, dirs, c2w, coeffs + (size_t)i * nb * 3, colors);
+    if constexpr (!STAGED) {
+        if (i >= n) return;
+        constexpr int kBytes = 3 * (D + 1) * (D + 1) * (int)sizeof(CT);
+        uint32_t w[(kBytes + 3) / 4];
+        w[(kBytes + 3) / 4 - 1] = 0;
+        __builtin_memcpy(w, coeffs + (size_t)i * nb * 3, kBytes);
+        sh_color<D>(i, dirs, c2w, RowWords<CT>{w}, colors);
         return;
     }
     const int R = 3 * nb * (int)sizeof(CT) / 4;  // words of a row
@@ -122,11 +130,7 @@ __global__ __launch_bounds__(256) void k_sh_forward(int n, int nb, const float* 
     }
     __syncthreads();
     if (i >= n) return;
-    const uint32_t* row = coef_stage + threadIdx.x * RS;
-    if constexpr (sizeof(CT) == 4)
-        sh_color<D>(i, dirs, c2w, reinterpret_cast<const float*>(row), colors);
-    else
-        sh_color<D>(i, dirs, c2w, Bf16Words{row}, colors);
+    sh_color<D>(i, dirs, c2w, RowWords<CT>{coef_stage + threadIdx.x * RS}, colors);
 }
 
 // v_coeffs[k][c] = basis_k * v_colors[c] for k < bases(D), zero above
@@ -220,9 +224,11 @@ static hipError_t sh_forward_t(int n, int degree, int degrees_to_use, const floa
     const size_t lds = (size_t)256 * ((bytes / 4) | 1) * 4;
     const bool staged =
         bytes % 4 == 0 && (reinterpret_cast<uintptr_t>(coeffs) & 15) == 0 && lds <= 65536;
-    const size_t sh = staged ? lds : 0;
-#define GSTEX_SHF(D) \
-    k_sh_forward<D, CT><<<g, 256, sh, stream>>>(n, nb, dirs, c2w, coeffs, colors, staged)
+#define GSTEX_SHF(D)                                                                           \
+    if (staged)                                                                                \
+        k_sh_forward<D, CT, true><<<g, 256, lds, stream>>>(n, nb, dirs, c2w, coeffs, colors);  \
+    else                                                                                       \
+        k_sh_forward<D, CT, false><<<g, 256, 0, stream>>>(n, nb, dirs, c2w, coeffs, colors)
     switch (degrees_to_use) {
         case 0: GSTEX_SHF(0); break;
         case 1: GSTEX_SHF(1); break;
