@@ -21,8 +21,9 @@ namespace gstex {
 // and float64 edge-on code for the common settings; MODE 1 keeps all of it;
 // MODE 2 is MODE 0 plus the float64 edge-on solve.  TB selects bfloat16
 // texels.  CM <= 4 is the exact channel count; above 4 it is a runtime count.
-// The plain kernels for CM <= 4 are held to 96 VGPRs (5 waves per SIMD), which
-// they need at most one register more than, those for a runtime count to 128.
+// The plain kernels for CM <= 4 are held to 96 VGPRs (5 waves per SIMD; with
+// three channels 2 of them and 32 SGPRs spill, with four 10 and 86), those for a
+// runtime count to 128.
 //
 // Texel gradients of the window route over the R x Q texels from chart row
 // ou, column ov (R, Q <= 3): window tap (row r, column q) has weight
