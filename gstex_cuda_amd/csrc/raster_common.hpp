@@ -937,17 +937,30 @@ inline RasterArgs make_raster_args(const RasterCall& c, const float* records) {
 // One, two and four channels, the blur and bfloat16 gain as much or more (256 to
 // 1350 tiles: both together 1.2 to 2.3 times as fast).
 //
-// The narrow backward holds a 4x4 texel window of a chart in LDS and four or more
-// whole charts a batch; what exceeds these goes out tap by tap, which costs as
-// the texel values that the lists name: entries times the mean values of a
-// chart.  Up to kNarrowBackwardValues of them it is no slower (charts sized by
-// area, 920 tiles, backward alone: 150K entries of 24 values a chart 366 against
-// 253 us, 70K of 48 462 against 378, 31K of 96 320 against 312); above it 150K of 48
-// 422 against 598, 70K of 96 526 against 675 and, 16x16 texels each, 136K of 768
-// 681 against 1707.
-constexpr int kNarrowTiles = 1400;
+// The narrow backward holds a 4x4 texel window of a chart in LDS and a pool of
+// 3,072 values for the whole charts of a batch; what exceeds these goes out tap by
+// tap, which costs as the texel values that the lists name: entries times the mean
+// values of a chart.  Up to kNarrowBackwardValues of them it is no slower (charts
+// sized by area, 920 tiles, backward alone: 150K entries of 24 values a chart 366
+// against 253 us, 70K of 48 462 against 378, 31K of 96 320 against 312); above it
+// 150K of 48 422 against 598, 70K of 96 526 against 675 and, 16x16 texels each, 136K
+// of 768 681 against 1707.  Small charts of one size (the texels a multiple of the
+// Gaussians, up to kNarrowChartOneSize values) leave the pool enough room at any
+// count: 4x4 texels of three channels, 608 tiles, 300K entries 362 against 235 us,
+// 920 tiles, 296K 329 against 251; 6x6 texels, 920 tiles, 296K 366 against 329.  So
+// do means of up to kNarrowChartMean values: charts of 4 texels of three channels
+// sized by area, 608 tiles, 419K 390 against 295.
+// On grids of over kNarrowManyTiles tiles there is less to gain: fewer entries
+// (kNarrowManyTilesIds; 1350 tiles, 419K of 12 values 305 against 343) and the
+// bound for every mean; and with under six entries a tile most blocks have next to
+// nothing to do and their set-up decides (1350 tiles, 4.5K entries of 12 values 39
+// against 50 us; but 1125 tiles, 8.4K 64 against 50).  Above kNarrowSparseTiles,
+// charts of several sizes need twelve (1350 tiles, 9.8K entries of 36 values 68
+// against 83; 29K 166 against 129).
+constexpr int kNarrowTiles = 1400, kNarrowManyTiles = 1000, kNarrowSparseTiles = 1200;
 constexpr int kNarrowForwardIds = 600000;
-constexpr int kNarrowBackwardIds = 450000;
+constexpr int kNarrowBackwardIds = 450000, kNarrowManyTilesIds = 300000;
+constexpr int kNarrowChartOneSize = 112, kNarrowChartMean = 16;
 constexpr double kNarrowBackwardValues = 4.5e6;
 bool raster_forward_is_narrow(const RasterArgs& a);
 bool raster_backward_is_narrow(const RasterArgs& a);

@@ -993,8 +993,17 @@ bool raster_forward_is_narrow(const RasterArgs& a) {
     return narrow_supported(a) && a.num_ids <= kNarrowForwardIds;
 }
 bool raster_backward_is_narrow(const RasterArgs& a) {
-    return narrow_supported(a) && a.num_ids <= kNarrowBackwardIds &&
-           (double)a.num_ids * a.channels * a.num_texels <= kNarrowBackwardValues * a.num_points;
+    if (!narrow_supported(a)) return false;
+    const int tiles = a.tiles_x * a.tiles_y;
+    const bool many = tiles > kNarrowManyTiles;
+    if (a.num_ids > (many ? kNarrowManyTilesIds : kNarrowBackwardIds)) return false;
+    const double chart = (double)a.channels * a.num_texels / a.num_points;  // mean values
+    const bool one_size = a.num_texels % a.num_points == 0 && chart <= kNarrowChartOneSize;
+    if (many && a.num_ids < (one_size || tiles <= kNarrowSparseTiles ? 6 : 12) * tiles)
+        return false;
+    if (one_size) return true;
+    if (!many && chart <= kNarrowChartMean) return true;
+    return a.num_ids * chart <= kNarrowBackwardValues;
 }
 
 template <int CM>
